@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define TFD_ABI_VERSION 16
+#define TFD_ABI_VERSION 17
 
 /* gemv prologues / epilogues */
 #define TFD_PRO_PLAIN 0  /* x used as given */
@@ -264,6 +264,48 @@ int tfd_finalize_rows(const int32_t* pick, int rows, const int32_t* inp, int ld_
 /* Embedding rows of ids[0..rows) (Qwen3_1_7B.embed per sequence, ref_src/model.py:279-287). */
 int tfd_embed_rows_bf16(const void* table, const int64_t* ids, void* out, int ldo, int rows,
                         int hidden, int vocab, int32_t* err, void* stream);
+
+/* ---- prompt passes: many prompt rows through a layer at once ------------------
+ * M rows of one or several sequences; row m is position pos[m] of sequence seq[m]
+ * (page-table row seq[m]).  Activations that feed a GEMM are in PANEL ORDER: 32-row
+ * panels, each in the skinny GEMMs' operand order, panel p at p * 32 * K (buffers hold
+ * ceil(M/32) * 32 * K bf16).  Replaces walking a prompt step by step
+ * (fast/engine.py:261-262); the semantics are ref_src/model.py:125-234 per position,
+ * the batched form the reference's placed fixture
+ * (tests/fixtures/placed/qwen3_1_7b_pd.py:55-230). */
+#define TFD_PANEL_PARTIAL 0 /* out f32 [slices][M][N]: K-split partial sums */
+#define TFD_PANEL_SWIGLU 1  /* out panel order [M][N/2] (one slice only) */
+/* K slices tfd_panel_gemm_bf16 uses for a shape (0: a shape it does not take). */
+int tfd_panel_gemm_slices(int M, int K, int N);
+/* Y[m][n] = sum_k X[m][k] W[n][k], X in panel order, W packed by tfd_pack_skinny_bf16,
+ * f32 sums; K % 256 == 0, N % 4 == 0.  TFD_PANEL_SWIGLU needs one slice and
+ * N/2 % 32 == 0: rows of W are (gate_i, up_i) pairs. */
+int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int epilogue,
+                        void* out, void* stream);
+/* SwiGLU over TFD_PANEL_PARTIAL sums of a gate/up projection -> panel order [M][N/2]. */
+int tfd_panel_swiglu(const float* part, int slices, int M, int N, void* out, void* stream);
+/* h = bf16(resid + bf16(sum of slices)) per row ([M][n], to h_out unless NULL; slices 0:
+ * h = resid) and its RMSNorm (tfd_rmsnorm_bf16's rounding) in panel order.  n % 32 == 0,
+ * n <= 8192. */
+int tfd_panel_add_norm(const float* part, int slices, const void* resid, void* h_out,
+                       const void* gamma, void* norm_out, int M, int n, float eps, void* stream);
+/* From the q/k/v partial sums: per-head RMSNorm and RoPE; q_out [M][heads * head_dim] bf16
+ * = bf16(q_rope * scale); k_rope and v written at pos[m] of sequence seq[m]'s pages. */
+int tfd_panel_qkv_append(const float* part, int slices, int M, int heads, int kv_heads,
+                         int head_dim, const void* gamma_q, const void* gamma_k,
+                         const void* cos_table, const void* sin_table, int rope_rows,
+                         const int32_t* pos, const int32_t* seq, const int32_t* page_table,
+                         int max_pages, void* k_pool, void* v_pool, int num_pages, float scale,
+                         float eps, void* q_out, int32_t* err, void* stream);
+/* Rows of an attention tile for `group` query heads per kv head. */
+int tfd_panel_attn_rows(int group);
+/* Causal attention of the rows over their sequences' pages (appended before the call).
+ * tiles int32 [ntiles][4]: first row, rows (up to tfd_panel_attn_rows), sequence, the
+ * first row's position; a tile's rows are consecutive positions.  out: panel order
+ * [M][heads * head_dim].  (head_dim, group) of (128, 2), (64, 2) or (128, 1). */
+int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, int kv_heads,
+                   int head_dim, const int32_t* page_table, int max_pages, const void* k_pool,
+                   const void* v_pool, int num_pages, void* out, int32_t* err, void* stream);
 
 /* ---- persistent decode step ------------------------------------------------
  * One cooperative launch runs `steps` whole decode steps (every layer, the head,

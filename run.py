@@ -225,8 +225,8 @@ def main(argv: list[str] | None = None) -> int:
                     help="Qwen3: prompt positions the engine reserves")
     ap.add_argument("--seed", type=int, default=0, help="weights / random prompt seed")
     ap.add_argument("--prefill", action="store_true",
-                    help="Qwen3: fill the prompt's cache in batched passes (32 positions per "
-                         "pass) instead of walking it one decode step per token")
+                    help="Qwen3: fill the prompt's cache in batched passes (up to 4,096 "
+                         "positions each) instead of walking it one decode step per token")
     ap.add_argument("--sample", action="store_true",
                     help="draw tokens instead of taking the largest logit (the model's "
                          "reference defaults unless the flags below say otherwise)")

@@ -1,0 +1,185 @@
+"""Prompt-pass kernels (csrc/prefill.hip) against plain f32 references, at the
+sizes where tiles and passes end, and the cut of prompts into passes (CPU)."""
+import pytest
+import torch
+
+from tilefoundry_amd import _lib
+from tilefoundry_amd.qwen3.prefill import plan_passes
+
+
+def panels(x):
+    """[M][K] rows in panel order (32-row panels in operand order, zero padded)."""
+    M, K = x.shape
+    P = -(-M // 32)
+    z = torch.zeros(P * 32, K, device=x.device, dtype=x.dtype)
+    z[:M] = x
+    return z.view(P, 2, 16, K // 32, 4, 8).permute(0, 3, 1, 4, 2, 5).contiguous().reshape(-1)
+
+
+def unpanel(flat, M, K):
+    P = -(-M // 32)
+    return flat[:P * 32 * K].view(P, K // 32, 2, 4, 16, 8).permute(0, 2, 4, 1, 3, 5).reshape(
+        P * 32, K)[:M]
+
+
+@pytest.mark.parametrize("lens,max_rows,tile", [
+    ([1], 4096, 64), ([64, 65, 1], 4096, 64), ([130, 7, 300], 100, 64), ([33, 33, 33], 32, 128),
+])
+def test_plan_passes_covers_every_row_once(lens, max_rows, tile):
+    segments = [([1000 * b + i for i in range(n)], 5 * b, b) for b, n in enumerate(lens)]
+    seen = []
+    for ids, pos, seqs, tiles in plan_passes(segments, max_rows, tile):
+        assert 0 < len(ids) <= max_rows and len(ids) == len(pos) == len(seqs)
+        rows = []
+        for row0, n, seq, p0 in tiles:
+            assert 0 < n <= tile
+            assert seqs[row0:row0 + n] == [seq] * n
+            assert pos[row0:row0 + n] == list(range(p0, p0 + n))
+            rows += range(row0, row0 + n)
+        assert sorted(rows) == list(range(len(ids)))
+        assert [t[3] + t[1] for t in tiles] == sorted((t[3] + t[1] for t in tiles), reverse=True)
+        seen += list(zip(seqs, pos, ids))
+    # each sequence's rows in the order of its positions, every one once
+    for b, (tokens, start, _) in enumerate(segments):
+        mine = [(p, t) for s, p, t in seen if s == b]
+        assert mine == [(start + i, t) for i, t in enumerate(tokens)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 31, 33, 64, 97, 128, 129, 300, 1100])
+@pytest.mark.parametrize("K,N", [(256, 768), (768, 256), (2048, 1056), (6144, 2048), (512, 40)])
+def test_panel_gemm(gpu_device, M, K, N):
+    """f32 sums of exact bf16 products: |error| <= K 2^-24 sum|x w| for any order."""
+    L = _lib.lib()
+    s = torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=gpu_device).manual_seed(M * 7 + K)
+    x = torch.randn(M, K, generator=g, device=gpu_device).to(torch.bfloat16)
+    w = torch.randn(N, K, generator=g, device=gpu_device).to(torch.bfloat16)
+    packed = torch.empty(-(-N // 16) * 16 * K, device=gpu_device, dtype=torch.bfloat16)
+    L.tfd_pack_skinny_bf16(w.data_ptr(), K, N, K, packed.data_ptr(), s)
+    xp = panels(x)
+    slices = L.tfd_panel_gemm_slices(M, K, N)
+    assert slices >= 1 and (K // 32) % slices == 0
+    part = torch.full((slices, M, N), float("nan"), device=gpu_device)
+    L.tfd_panel_gemm_bf16(xp.data_ptr(), packed.data_ptr(), M, K, N, _lib.PANEL_PARTIAL,
+                          part.data_ptr(), s)
+    want = x.double() @ w.double().t()
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    assert ((part.double().sum(0) - want).abs() <= bound).all()
+    if N % 64:
+        return
+    # SwiGLU, from the partial sums (added in slice order, as the kernel adds them) and
+    # (one slice) from the GEMM itself: two bf16 roundings after the sums, which an ulp
+    # of exp may settle another way
+    r = part[0].clone()
+    for sl in range(1, slices):
+        r += part[sl]
+    r = r.to(torch.bfloat16).float()
+    act = torch.nn.functional.silu(r[:, 0::2]).to(torch.bfloat16).float() * r[:, 1::2]
+    out = torch.zeros(-(-M // 32) * 32 * (N // 2), device=gpu_device, dtype=torch.bfloat16)
+    L.tfd_panel_swiglu(part.data_ptr(), slices, M, N, out.data_ptr(), s)
+    assert ((unpanel(out, M, N // 2).float() - act).abs() <= 2.0 ** -6 * act.abs() + 1e-6).all()
+    if slices == 1:
+        two = torch.zeros_like(out)
+        L.tfd_panel_gemm_bf16(xp.data_ptr(), packed.data_ptr(), M, K, N, _lib.PANEL_SWIGLU,
+                              two.data_ptr(), s)
+        assert torch.equal(two, out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("slices,M,n", [(0, 1, 256), (1, 33, 2048), (3, 65, 2048), (2, 5, 4096)])
+def test_panel_add_norm(gpu_device, slices, M, n):
+    """The residual sum rounds once more (equal bits: the slices add in order); the
+    norm is bf16(bf16(h r) gamma), r within f32 rounding: one ulp of either."""
+    L = _lib.lib()
+    g = torch.Generator(device=gpu_device).manual_seed(n + M)
+    part = torch.randn(max(slices, 1), M, n, generator=g, device=gpu_device)
+    resid = torch.randn(M, n, generator=g, device=gpu_device).to(torch.bfloat16)
+    gamma = (1 + 0.1 * torch.randn(n, generator=g, device=gpu_device)).to(torch.bfloat16)
+    h = torch.zeros_like(resid)
+    out = torch.zeros(-(-M // 32) * 32 * n, device=gpu_device, dtype=torch.bfloat16)
+    L.tfd_panel_add_norm(part.data_ptr(), slices, resid.data_ptr(), h.data_ptr(),
+                         gamma.data_ptr(), out.data_ptr(), M, n, 1e-6,
+                         torch.cuda.current_stream().cuda_stream)
+    want = resid
+    if slices:
+        y = part[0].clone()
+        for sl in range(1, slices):
+            y += part[sl]
+        want = (resid.float() + y.to(torch.bfloat16).float()).to(torch.bfloat16)
+    assert torch.equal(h, want)
+    f = want.float()
+    r = torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-6)
+    norm = (f * r).to(torch.bfloat16).float() * gamma.float()
+    assert ((unpanel(out, M, n).float() - norm).abs() <= 2.0 ** -7 * norm.abs() + 1e-6).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,G", [(128, 2), (64, 2), (128, 1)])
+@pytest.mark.parametrize("segs", [[(0, 1)], [(0, 64), (63, 1)], [(0, 200), (70, 129), (128, 3)]])
+def test_panel_attn(gpu_device, D, G, segs):
+    """(first position, rows) segments over filled pages against f32 softmax.  Scores
+    are rounded to bf16 (|s| < 8 here: 2^-6 absolute), probabilities twice and the
+    output three times at 2^-9: 3e-2 of the largest |value| bounds every output."""
+    L = _lib.lib()
+    HKV = 2
+    heads = HKV * G
+    g = torch.Generator(device=gpu_device).manual_seed(D + len(segs))
+    pages = -(-max(p + n for p, n in segs) // 16) + 1
+    B = len(segs)
+    table = torch.randperm(B * pages, generator=torch.Generator().manual_seed(1)).view(
+        B, pages).to(torch.int32).to(gpu_device)
+    bf = torch.bfloat16
+    k = torch.randn(B * pages, HKV, 16, D, generator=g, device=gpu_device).to(bf)
+    v = torch.randn(B * pages, HKV, 16, D, generator=g, device=gpu_device).to(bf)
+    M = sum(n for _, n in segs)
+    q = (torch.randn(M, heads, D, generator=g, device=gpu_device) * D ** -0.5).to(bf)
+    qt = L.tfd_panel_attn_rows(G)
+    tiles, row = [], 0
+    for b, (p0, n) in enumerate(segs):
+        tiles += [(row + t, min(qt, n - t), b, p0 + t) for t in range(0, n, qt)]
+        row += n
+    td = torch.tensor(tiles, dtype=torch.int32, device=gpu_device)
+    out = torch.zeros(-(-M // 32) * 32 * heads * D, device=gpu_device, dtype=bf)
+    err = torch.zeros(1, device=gpu_device, dtype=torch.int32)
+    L.tfd_panel_attn(q.data_ptr(), td.data_ptr(), len(tiles), heads, HKV, D, table.data_ptr(),
+                     pages, k.data_ptr(), v.data_ptr(), B * pages, out.data_ptr(),
+                     err.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    got = unpanel(out, M, heads * D).float().view(M, heads, D)
+    assert int(err.item()) == 0
+    row = 0
+    for b, (p0, n) in enumerate(segs):
+        p = torch.arange(p0 + n, device=gpu_device)
+        kc, vc = (t[table[b].long()[p // 16], :, p % 16].float().repeat_interleave(G, 1)
+                  for t in (k, v))
+        s = torch.einsum("mhd,phd->hmp", q[row:row + n].float(), kc)
+        late = p[None, :] > (p0 + torch.arange(n, device=gpu_device))[:, None]
+        a = torch.softmax(s.masked_fill(late, float("-inf")), -1)
+        want = torch.einsum("hmp,phd->mhd", a, vc)
+        assert (got[row:row + n] - want).abs().max() <= 3e-2 * want.abs().max()
+        row += n
+
+
+@pytest.mark.gpu
+def test_passes_cut_anywhere_fill_the_same_cache(gpu_device, monkeypatch):
+    """Three prompts in one pass and in passes of 64 rows: the same caches to the
+    bf16 bar (other GEMM shapes, other f32 orders)."""
+    from tests._parity import assert_close_bf16
+    from tests.test_gpu_engine import SMALL, _prompt
+    from tilefoundry_amd.qwen3 import prefill, synthetic_weights
+    from tilefoundry_amd.qwen3.batch_engine import BatchEngine
+
+    w = synthetic_weights(SMALL, seed=1, norms="ones")
+    prompts = [_prompt(n, SMALL.vocab_size, seed=n) for n in (90, 2, 71)]
+    eng = BatchEngine(SMALL, w, batch=3, device=gpu_device, max_new=8, prompt_room=96)
+    eng.kpool.zero_()                       # the capture's own steps left rows behind
+    eng.vpool.zero_()
+    eng.prefill(prompts)
+    k, v = eng.kpool.clone(), eng.vpool.clone()
+    monkeypatch.setattr(prefill, "MAX_PASS", 64)
+    eng.kpool.zero_()
+    eng.vpool.zero_()
+    eng.prefill(prompts)
+    eng.check_errors()
+    assert_close_bf16(eng.kpool, k, max_rel=2e-2, name="k")
+    assert_close_bf16(eng.vpool, v, max_rel=2e-2, name="v")

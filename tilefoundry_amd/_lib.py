@@ -13,7 +13,7 @@ from pathlib import Path
 
 from .build import LIB
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 PRO_PLAIN, PRO_NORM = 0, 1
 EPI_STORE, EPI_RESID, EPI_SWIGLU, EPI_LOGITS, EPI_RESID_F32 = 0, 1, 2, 3, 4
@@ -25,6 +25,7 @@ NOALLOC_SCRATCH_FLOATS = SKINNY_COUNTERS + (1 << 21)   # tfd_gemm_skinny_bf16_no
 ARGMAX_WORK = 128           # int32 per row of tfd_argmax_rows' two-stage work buffer
 ATTN_SPLIT = 64
 ROUTE_SOFTMAX_TOPK, ROUTE_TOPK_SOFTMAX = 0, 1
+PANEL_PARTIAL, PANEL_SWIGLU = 0, 1   # tfd_panel_gemm_bf16's outputs
 
 
 def moe_group_words(experts: int, rows: int) -> int:
@@ -83,6 +84,13 @@ SIGNATURES: dict[str, list] = {
     "tfd_argmax_rows": [P, I, I, I, P, P, P],
     "tfd_finalize_rows": [P, I, P, I, P, P, P, P, I, I, P, P, I, I, I, P, P],
     "tfd_embed_rows_bf16": [P, P, P, I, I, I, I, P, P],
+    "tfd_panel_gemm_slices": [I, I, I],
+    "tfd_panel_gemm_bf16": [P, P, I, I, I, I, P, P],
+    "tfd_panel_swiglu": [P, I, I, I, P, P],
+    "tfd_panel_add_norm": [P, I, P, P, P, P, I, I, F, P],
+    "tfd_panel_qkv_append": [P, I, I, I, I, I, P, P, P, P, I, P, P, P, I, P, P, I, F, F, P, P, P],
+    "tfd_panel_attn_rows": [I],
+    "tfd_panel_attn": [P, P, I, I, I, I, P, I, P, P, I, P, P, P],
     "tfd_decode_persistent": [P, I, I, P],
     "tfd_decode_persistent_grid": [],
     "tfd_decode_xcd": [P, P, I, P],
@@ -114,7 +122,8 @@ SIGNATURES: dict[str, list] = {
     "tfd_moe_experts_small": [P, P],
 }
 RESTYPES = {"tfd_last_error": ctypes.c_char_p, "tfd_sample_work_bytes": ctypes.c_int64}
-UNCHECKED = {"tfd_abi_version", "tfd_decode_persistent_grid"}
+UNCHECKED = {"tfd_abi_version", "tfd_decode_persistent_grid", "tfd_panel_gemm_slices",
+             "tfd_panel_attn_rows"}
 
 
 class TfdLayer(ctypes.Structure):

@@ -1,0 +1,715 @@
+// Prompt passes: hundreds to thousands of prompt rows through a layer at once.
+//
+// A decode step's kernels are made for at most 32 rows: a prompt taken through
+// them reads every weight once per 32 tokens and every cached key once per row.
+// Here a pass takes all its rows (up to 4,096, of one or several sequences)
+// through each layer together:
+//   k_gemm_panels    projections: weights in the skinny GEMMs' packed blocks,
+//                    activations in panel order (panel.h), f32 partial sums or a
+//                    SwiGLU epilogue
+//   k_panel_qkv      q/k norm, RoPE, cache append
+//   k_panel_attn     causal attention over the paged cache on the matrix cores
+//   k_panel_add_norm residual add and the next RMSNorm
+//   k_panel_swiglu   SwiGLU over K-split gate/up sums
+// Rounding points are the HIR's (ref_src/model.py:125-234); attention's two
+// products are exact, as the reference's own fast path takes them (T.gemm,
+// examples/qwen3_1_7b-tilelang/fast/kernels.py:418-501).
+
+#include <type_traits>
+
+#include "host_common.h"
+#include "panel.h"
+#include "tf_decode.h"
+
+using namespace tfd;
+using namespace tfd_host;
+
+namespace {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr float kNegInf = -__builtin_huge_valf();
+
+__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+
+// One 16-row x 32-k block of packed weights as a matrix-core operand.
+__device__ __forceinline__ u32x4 weight_block(const bf16* W, int64_t block, int lane) {
+  return load16(W + block * 512 + lane * 8);
+}
+
+// ---------------------------------------------------------------------------
+// Y[m][n] = sum_k X[m][k] W[n][k] for M rows in panel order.  A block of four
+// waves takes TM x 16 rows and 4 x TN x 16 columns over its K slice; a wave owns
+// TN column tiles for all the block's rows.  The weights go straight from memory
+// to the wave's registers (packed blocks are matrix-core operands as they lie,
+// and no other wave of the block reads them), DB K steps ahead; the rows, which
+// every wave reads, pass through LDS, KC steps at a time in two buffers.
+//
+// The weight is the A operand and the row the B operand, so a lane ends up with
+// four consecutive columns of one row: a partial is one 16-byte store, and a
+// SwiGLU's (gate, up) pairs sit in one lane.
+//
+// Bound: at thousands of rows the matrix cores and LDS (a wave reads eight row
+// blocks per 32 matrix products), below 128 rows the weights' stream.  Measured,
+// weights cold (M x K x N): 4,000 x 2048 x 12288 266 us (757 TFLOP/s), 4,000 x 6144 x
+// 2048 117 us (863); 91 x 2048 x 12288 17.8 us (2.8 TB/s of weights); 17 x 2048 x
+// 4096 5.3 us.  The skinny GEMM took 126 launches for the 4,000 rows, 15 us each for
+// 2048 x 12288.
+//
+// grid: 8 x ceil(tiles / 8) blocks.  Consecutive tiles (eight row blocks by a
+// few column blocks) go to one XCD, so that the operands its blocks share stay in
+// its L2.
+// ---------------------------------------------------------------------------
+enum PanelEpi { kPanPartial = 0, kPanSwiglu = 1 };
+
+template <int TM, int TN, int KC, int DB, int kEpi>
+__global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__ X,
+                                                        const bf16* __restrict__ W, int M, int K,
+                                                        int N, int slices,
+                                                        void* __restrict__ out) {
+  constexpr int kPasses = KC * TM / 4;       // 16-byte loads per thread of one LDS chunk
+  static_assert(DB % KC == 0 && TM % 2 == 0 && KC * TM % 4 == 0, "tile shape");
+  __shared__ __align__(16) uint8_t xs[2][KC * TM * 1024];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int nm = (M + TM * 16 - 1) / (TM * 16);
+  const int ntiles = (N + 15) / 16;
+  const int nn = (ntiles + 4 * TN - 1) / (4 * TN);
+  const int total = nm * nn * slices, per = (total + 7) / 8;
+  const int g = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || g >= total) return;
+  const int slice = g / (nm * nn), rest = g % (nm * nn);
+  const int grp = rest / (8 * nn), within = rest % (8 * nn);
+  const int gm = min(8, nm - grp * 8);
+  const int mb = grp * 8 + within % gm, nb = within / gm;
+
+  const int ksteps = K / 32;
+  const int steps = ksteps / slices, s0 = slice * steps;
+  const int panels = (M + 31) / 32;
+
+  // the block's rows: this thread's 16-byte pieces of a chunk (2 KiB per panel
+  // and step; a panel past the last one repeats it, its rows are not stored)
+  const bf16* xsrc[kPasses];
+#pragma unroll
+  for (int q = 0; q < kPasses; ++q) {
+    const int blk = q * 2 + (tid >> 7);
+    const int st = blk / (TM / 2), pn = min(mb * (TM / 2) + blk % (TM / 2), panels - 1);
+    xsrc[q] = X + ((int64_t)pn * ksteps + s0 + st) * 1024 + (tid & 127) * 8;
+  }
+  int64_t wt[TN];
+#pragma unroll
+  for (int t = 0; t < TN; ++t)
+    wt[t] = (int64_t)min((nb * 4 + wave) * TN + t, ntiles - 1) * ksteps + s0;
+
+  u32x4 xr[kPasses], b[DB][TN];
+  auto load_x = [&](int step) {
+#pragma unroll
+    for (int q = 0; q < kPasses; ++q) xr[q] = load16(xsrc[q] + (int64_t)step * 1024);
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < kPasses; ++q)
+      *reinterpret_cast<u32x4*>(&xs[buf][q * 4096 + tid * 16]) = xr[q];
+  };
+  load_x(0);
+#pragma unroll
+  for (int u = 0; u < DB; ++u)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) b[u][t] = weight_block(W, wt[t] + u, lane);
+  f32x4 c[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) c[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  stage(0);
+  __syncthreads();
+  int cur = 0;
+  // DB steps from step k0 on; with kMore every slot is refilled behind its use
+  // and the next chunk of rows follows (the last body has nothing ahead)
+  auto body = [&](int k0, auto more) {
+#pragma unroll
+    for (int u0 = 0; u0 < DB; u0 += KC) {
+      constexpr bool kMore = decltype(more)::value;
+      const bool next = kMore || u0 + KC < DB;
+      if (next) load_x(k0 + u0 + KC);
+#pragma unroll
+      for (int v = 0; v < KC; ++v) {
+        const int u = u0 + v;
+        u32x4 a[TM];
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+          a[m] = *reinterpret_cast<const u32x4*>(&xs[cur][(v * TM + m) * 1024 + lane * 16]);
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+#pragma unroll
+          for (int m = 0; m < TM; ++m) c[m][t] = mfma(b[u][t], a[m], c[m][t]);
+        if (kMore)
+#pragma unroll
+          for (int t = 0; t < TN; ++t)
+            b[u][t] = weight_block(W, wt[t] + k0 + u + DB, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (next) {
+        cur ^= 1;
+        stage(cur);
+        __syncthreads();
+      }
+    }
+  };
+  for (int k0 = 0; k0 + DB < steps; k0 += DB) body(k0, std::true_type{});
+  body(steps - DB, std::false_type{});
+
+  const int r = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    const int row = (mb * TM + m) * 16 + r;
+    if (row >= M) continue;
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int n = ((nb * 4 + wave) * TN + t) * 16 + 4 * kq;
+      if (n >= N) continue;
+      if (kEpi == kPanSwiglu) {
+        const float g0 = rbf(c[m][t].x), u0 = rbf(c[m][t].y);
+        const float g1 = rbf(c[m][t].z), u1 = rbf(c[m][t].w);
+        *reinterpret_cast<uint32_t*>((bf16*)out + panel_off(row, n / 2, N / 2)) =
+            pack2(rbf(silu_f(g0)) * u0, rbf(silu_f(g1)) * u1);
+      } else {
+        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)slice * M + row) * N + n) = c[m][t];
+      }
+    }
+  }
+}
+
+// The sum of a value's K slices, in slice order, rounded once.
+__device__ __forceinline__ float slice_sum(const float* p, int64_t stride, int slices) {
+  float a = p[0];
+  for (int s = 1; s < slices; ++s) a += p[s * stride];
+  return rbf(a);
+}
+
+// ---------------------------------------------------------------------------
+// After the q/k/v projection (model.py:172-190, 339-352): per head RMSNorm and
+// RoPE of the queries (times the score scale) and keys, keys and values appended
+// at the row's position of its sequence's pages.  A wave per (row, head vector).
+// ---------------------------------------------------------------------------
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_panel_qkv(
+    const float* __restrict__ part, int slices, int M, int heads, int kv_heads,
+    const bf16* __restrict__ gq, const bf16* __restrict__ gk, const bf16* __restrict__ cos_t,
+    const bf16* __restrict__ sin_t, int rope_rows, const int* __restrict__ pos,
+    const int* __restrict__ seq, const int* __restrict__ page_table, int max_pages,
+    bf16* __restrict__ kpool, bf16* __restrict__ vpool, int num_pages, float scale, float eps,
+    bf16* __restrict__ q_out, int* err) {
+  constexpr int kHalf = D / 2;
+  const int m = blockIdx.x, lane = threadIdx.x & (kWave - 1);
+  const int v = blockIdx.y * kWavesPerBlock + threadIdx.x / kWave;
+  if (v >= heads + 2 * kv_heads) return;
+  const int N = (heads + 2 * kv_heads) * D;
+  const int P = pos[m];
+  const bool isq = v < heads, isv = v >= heads + kv_heads;
+  if (P < 0 || P >= rope_rows || P >= max_pages * kPage) {
+    if (lane == 0) raise_error(err, kErrPosRange);
+    return;
+  }
+  const bool act = lane < kHalf;
+  const int li = act ? lane : 0;
+  const float* x = part + (int64_t)m * N + v * D;
+  const int64_t stride = (int64_t)M * N;
+  const float x0 = act ? slice_sum(x + li, stride, slices) : 0.f;
+  const float x1 = act ? slice_sum(x + li + kHalf, stride, slices) : 0.f;
+  float o0 = x0, o1 = x1;
+  if (!isv) {
+    const bf16* gam = isq ? gq : gk;
+    float ss = x0 * x0;
+    ss += x1 * x1;
+    ss = wave_sum(ss);
+    const float r = 1.0f / sqrtf(ss / (float)D + eps);
+    const int64_t row = (int64_t)P * D;
+    const float n0 = rbf(rbf(x0 * r) * bf2f(gam[li]));
+    const float n1 = rbf(rbf(x1 * r) * bf2f(gam[li + kHalf]));
+    o0 = rbf(n0 * bf2f(cos_t[row + li]) + (-n1) * bf2f(sin_t[row + li]));
+    o1 = rbf(n1 * bf2f(cos_t[row + li + kHalf]) + n0 * bf2f(sin_t[row + li + kHalf]));
+  }
+  if (!act) return;
+  if (isq) {
+    bf16* q = q_out + ((int64_t)m * heads + v) * D;
+    q[li] = f2bf(o0 * scale);
+    q[li + kHalf] = f2bf(o1 * scale);
+    return;
+  }
+  const int page = page_table[(int64_t)seq[m] * max_pages + P / kPage];
+  if (page < 0 || page >= num_pages) {
+    if (lane == 0) raise_error(err, kErrPageRange);
+    return;
+  }
+  const int h = isv ? v - heads - kv_heads : v - heads;
+  bf16* pool = isv ? vpool : kpool;
+  bf16* o = pool + (((int64_t)page * kv_heads + h) * kPage + P % kPage) * D;
+  o[li] = f2bf(o0);
+  o[li + kHalf] = f2bf(o1);
+}
+
+// ---------------------------------------------------------------------------
+// Causal attention of a prompt pass (model.py:190-212) over the paged cache,
+// which already holds the pass's own keys and values.
+//
+// A block takes one tile of consecutive rows of a sequence (128 / G of them) and
+// one kv head: 128 (query head, row) columns, 32 per wave, past the context in
+// tiles of 64 positions.  S^T = K Q^T puts four consecutive positions of one
+// column in a lane; packed, that is the B operand of O^T = V^T P^T as it stands
+// if V^T's positions are stored in the same order, so the probabilities never
+// leave their lane.  K and V tiles are read once per block, prefetched into
+// registers while the tile before is used, V transposed on its way into LDS.
+//
+// Bound: LDS reads and the softmax's VALU work, about equally.  The decode kernels
+// it takes the place of re-read every cached key for each row: a 4,001-token prompt
+// through eight layers took 123.0 ms, with these kernels 7.7 ms; 91 tokens 2.18 and
+// 1.05 ms, eight prompts of 88-700 tokens 51.4 and 5.7 ms (each with one decode step).
+//
+// Rounding: s = bf16(q . k), p = bf16(exp(bf16(s - m))) against the running
+// maximum m (the HIR's final maximum from the tile that holds it on; sums and
+// outputs are rescaled in f32), the row's own key as its own term at the end
+// (model.py:198-212).
+// ---------------------------------------------------------------------------
+struct PanelTile {
+  int row0, rows, seq, pos0;
+};
+
+template <int D, int G>
+__global__ __launch_bounds__(kBlock) void k_panel_attn(
+    const bf16* __restrict__ q, const PanelTile* __restrict__ tiles, int heads, int kv_heads,
+    const int* __restrict__ page_table, int max_pages, const bf16* __restrict__ kpool,
+    const bf16* __restrict__ vpool, int num_pages, bf16* __restrict__ out, int* err) {
+  constexpr int QT = 128 / G;                // rows of a tile
+  constexpr int DS = D / 32, DT = D / 16;    // k steps of q.k, 16-row tiles of V^T
+  constexpr int KS = D + 8, VS = 64 + 8;     // LDS row strides (bf16)
+  constexpr int kCh = D / 8;                 // 16-byte chunks of a head row
+  constexpr int kKPass = 64 * kCh / kBlock;  // K loads per thread and tile
+  constexpr int kVThr = 16 * kCh;            // threads that move V: 4 positions x 8 dims each
+  __shared__ __align__(16) bf16 ks[64 * KS];
+  __shared__ __align__(16) bf16 vt[D * VS];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int r = lane & 15, kq = lane >> 4;
+  const int h = blockIdx.x;
+  const PanelTile tl = tiles[blockIdx.y];
+  const int last = tl.pos0 + tl.rows - 1;    // the last row's position
+  if (tl.pos0 < 0 || last >= max_pages * kPage) {
+    if (tid == 0) raise_error(err, kErrPosRange);
+    return;
+  }
+  const int* pt = page_table + (int64_t)tl.seq * max_pages;
+  auto page_of = [&](int p) {                // positions past the pages re-read the last
+    const int pg = pt[min(p, max_pages * kPage - 1) / kPage];
+    if (pg >= 0 && pg < num_pages) return pg;
+    raise_error(err, kErrPageRange);
+    return 0;
+  };
+
+  // this wave's columns: c = 32 wave + 16 ct + r -> query head c / QT, row c % QT
+  u32x4 qf[2][DS];
+  int qpos[2];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    const int c = 32 * wave + 16 * ct + r;
+    const int row = min(c % QT, tl.rows - 1);
+    qpos[ct] = tl.pos0 + row;
+    const bf16* qp = q + ((int64_t)(tl.row0 + row) * heads + h * G + c / QT) * D;
+#pragma unroll
+    for (int s = 0; s < DS; ++s) qf[ct][s] = load16(qp + 32 * s + 8 * kq);
+  }
+
+  u32x4 kr[kKPass], vr[4];
+  const int vg = tid / kCh, vc = tid % kCh;  // V: position group of 4, 8-dim chunk
+  auto load_tile = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < kKPass; ++i) {
+      const int c = tid + i * kBlock, p = j0 + c / kCh;
+      kr[i] = load16(kpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
+                     (c % kCh) * 8);
+    }
+    if (kVThr == kBlock || tid < kVThr) {
+      const int p = j0 + 4 * vg;
+      const bf16* v0 = vpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
+                       vc * 8;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vr[i] = load16(v0 + i * D);
+    }
+  };
+  auto stage_tile = [&]() {
+#pragma unroll
+    for (int i = 0; i < kKPass; ++i) {
+      const int c = tid + i * kBlock;
+      *reinterpret_cast<u32x4*>(&ks[(c / kCh) * KS + (c % kCh) * 8]) = kr[i];
+    }
+    if (kVThr == kBlock || tid < kVThr) {
+      // positions in the order the probabilities come in: within 32, position
+      // 16 t + 4 g + e sits at 8 g + 4 t + e
+      const int at = 32 * (vg >> 3) + 8 * (vg & 3) + 4 * ((vg >> 2) & 1);
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t w0 = (d >> 1) == 0 ? vr[0].x : (d >> 1) == 1 ? vr[0].y : (d >> 1) == 2 ? vr[0].z : vr[0].w;
+        const uint32_t w1 = (d >> 1) == 0 ? vr[1].x : (d >> 1) == 1 ? vr[1].y : (d >> 1) == 2 ? vr[1].z : vr[1].w;
+        const uint32_t w2 = (d >> 1) == 0 ? vr[2].x : (d >> 1) == 1 ? vr[2].y : (d >> 1) == 2 ? vr[2].z : vr[2].w;
+        const uint32_t w3 = (d >> 1) == 0 ? vr[3].x : (d >> 1) == 1 ? vr[3].y : (d >> 1) == 2 ? vr[3].z : vr[3].w;
+        const u32x2 o = {__builtin_amdgcn_perm(w1, w0, sel), __builtin_amdgcn_perm(w3, w2, sel)};
+        *reinterpret_cast<u32x2*>(&vt[(vc * 8 + d) * VS + at]) = o;
+      }
+    }
+  };
+
+  f32x4 o[DT][2];
+  float mx[2] = {kNegInf, kNegInf}, sum[2] = {0.f, 0.f}, self[2] = {kNegInf, kNegInf};
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt][0] = o[dt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  load_tile(0);
+  for (int j0 = 0; j0 <= last; j0 += 64) {
+    stage_tile();
+    __syncthreads();
+    if (j0 + 64 <= last) load_tile(j0 + 64);
+    f32x4 st[4][2];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) st[p][0] = st[p][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < DS; ++s)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const u32x4 kf = *reinterpret_cast<const u32x4*>(&ks[(16 * p + r) * KS + 32 * s + 8 * kq]);
+        st[p][0] = mfma(kf, qf[0][s], st[p][0]);
+        st[p][1] = mfma(kf, qf[1][s], st[p][1]);
+      }
+    u32x4 pb[2][2];                          // the packed probabilities of 32 positions each
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) {
+      const int before = qpos[ct] - j0 - 4 * kq;   // position 16 p + e is past: 16 p + e < before
+      float tm = kNegInf;
+      if (j0 + 64 > tl.pos0) {               // a tile that reaches the diagonal
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float s = rbf(st[p][ct][e]);
+            if (16 * p + e == before) self[ct] = s;
+            if (16 * p + e <= before) tm = fmaxf(tm, s);
+            st[p][ct][e] = 16 * p + e < before ? s : kNegInf;
+          }
+      } else {
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            st[p][ct][e] = rbf(st[p][ct][e]);
+            tm = fmaxf(tm, st[p][ct][e]);
+          }
+      }
+      float lo, hi;
+      pair16(tm, lo, hi);
+      tm = fmaxf(lo, hi);
+      pair32(tm, lo, hi);
+      tm = fmaxf(lo, hi);
+      const float m1 = fmaxf(mx[ct], tm);
+      const float alpha = expf(mx[ct] - m1);
+      mx[ct] = m1;
+      sum[ct] *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[dt][ct][e] *= alpha;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        float pe[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pe[e] = rbf(expf(rbf(st[p][ct][e] - m1)));
+          sum[ct] += pe[e];
+        }
+        const uint32_t w0 = pack2(pe[0], pe[1]), w1 = pack2(pe[2], pe[3]);
+        if (p & 1) {
+          pb[p >> 1][ct].z = w0;
+          pb[p >> 1][ct].w = w1;
+        } else {
+          pb[p >> 1][ct].x = w0;
+          pb[p >> 1][ct].y = w1;
+        }
+      }
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u32x4 vf = *reinterpret_cast<const u32x4*>(&vt[(16 * dt + r) * VS + 32 * kk + 8 * kq]);
+        o[dt][0] = mfma(vf, pb[kk][0], o[dt][0]);
+        o[dt][1] = mfma(vf, pb[kk][1], o[dt][1]);
+      }
+    __syncthreads();
+  }
+
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct) {
+    const int c = 32 * wave + 16 * ct + r;
+    float lo, hi, l = sum[ct], sn = self[ct];
+    pair16(l, lo, hi);
+    l = lo + hi;
+    pair32(l, lo, hi);
+    l = lo + hi;
+    pair16(sn, lo, hi);
+    sn = fmaxf(lo, hi);
+    pair32(sn, lo, hi);
+    sn = fmaxf(lo, hi);
+    const float pn = rbf(expf(rbf(sn - mx[ct])));
+    const float total = rbf(rbf(l) + pn);
+    const int P = qpos[ct];
+    const bf16* vrow = vpool + (((int64_t)page_of(P) * kv_heads + h) * kPage + P % kPage) * D;
+    const int row = c % QT;
+    const int64_t m = tl.row0 + row;
+    const int k0 = (h * G + c / QT) * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const u32x2 vw = *reinterpret_cast<const u32x2*>(vrow + 16 * dt + 4 * kq);
+      const float vn[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
+      float y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = rbf(rbf(o[dt][ct][e]) + rbf(pn * vn[e])) / total;
+      if (row < tl.rows)
+        *reinterpret_cast<u32x2*>(out + panel_off(m, k0 + 16 * dt + 4 * kq, heads * D)) =
+            u32x2{pack2(y[0], y[1]), pack2(y[2], y[3])};
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// h = resid + bf16(sum of the slices), and the next RMSNorm of h in panel order
+// (model.py:125-137, 213-225).  A block per row; slices 0: h = resid as it is.
+// ---------------------------------------------------------------------------
+template <int kCh>
+__global__ __launch_bounds__(kBlock) void k_panel_add_norm(
+    const float* __restrict__ part, int slices, const bf16* resid, bf16* h_out,
+    const bf16* __restrict__ gamma, bf16* __restrict__ norm_out, int M, int n, float eps) {
+  __shared__ float red[kWavesPerBlock];
+  const int64_t m = blockIdx.x;
+  const int tid = threadIdx.x, nch = n / 8;
+  u32x4 x[kCh];
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < kCh; ++i) {
+    const int c = min(tid + i * kBlock, nch - 1);
+    const u32x4 rv = load16(resid + m * n + c * 8);
+    float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < slices; ++s) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(part + ((int64_t)s * M + m) * n + c * 8);
+      const f32x4 lo = p[0], hi = p[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        y[e] += lo[e];
+        y[e + 4] += hi[e];
+      }
+    }
+    const uint32_t w[4] = {rv.x, rv.y, rv.z, rv.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = slices ? pack2(bf_lo(w[e]) + rbf(y[2 * e]), bf_hi(w[e]) + rbf(y[2 * e + 1])) : w[e];
+    x[i] = u32x4{o[0], o[1], o[2], o[3]};
+    if (tid + i * kBlock < nch) {
+      if (h_out) *reinterpret_cast<u32x4*>(h_out + m * n + c * 8) = x[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = bf_lo(o[e]), b = bf_hi(o[e]);
+        ss += a * a;
+        ss += b * b;
+      }
+    }
+  }
+  ss = wave_sum(ss);
+  if ((tid & (kWave - 1)) == 0) red[tid / kWave] = ss;
+  __syncthreads();
+  ss = red[0];
+  for (int w = 1; w < kWavesPerBlock; ++w) ss += red[w];
+  const float rs = 1.0f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+  for (int i = 0; i < kCh; ++i) {
+    const int c = tid + i * kBlock;
+    if (c < nch)
+      *reinterpret_cast<u32x4*>(norm_out + panel_off(m, c * 8, n)) =
+          rms_norm_chunk(x[i], load16(gamma + c * 8), rs);
+  }
+}
+
+// SwiGLU of K-split gate/up sums: (gate, up) pairs in adjacent columns.
+__global__ __launch_bounds__(kBlock) void k_panel_swiglu(const float* __restrict__ part,
+                                                         int slices, int M, int N,
+                                                         bf16* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;   // four columns each
+  const int per = N / 4;
+  if (i >= (int64_t)M * per) return;
+  const int64_t m = i / per;
+  const int n = (int)(i % per) * 4;
+  f32x4 a = *reinterpret_cast<const f32x4*>(part + m * N + n);
+  for (int s = 1; s < slices; ++s)
+    a += *reinterpret_cast<const f32x4*>(part + ((int64_t)s * M + m) * N + n);
+  const float h0 = rbf(silu_f(rbf(a.x))) * rbf(a.y), h1 = rbf(silu_f(rbf(a.z))) * rbf(a.w);
+  *reinterpret_cast<uint32_t*>(out + panel_off(m, n / 2, N / 2)) = pack2(h0, h1);
+}
+
+// ---------------------------------------------------------------------------
+// Tile shape and K slices of a panel GEMM: 16-row tiles per block (every row up
+// to 128, else 128), column tiles per wave, and as few slices as give the chip's
+// compute units a block each.
+// ---------------------------------------------------------------------------
+struct PanelPlan {
+  int tm, tn, slices;
+};
+
+PanelPlan panel_plan(int M, int K, int N) {
+  PanelPlan p;
+  const int cus = compute_units(), ntiles = (N + 15) / 16, ksteps = K / 32;
+  p.tm = M <= 128 ? (M + 31) / 32 * 2 : 8;
+  const int nm = (M + p.tm * 16 - 1) / (p.tm * 16);
+  auto blocks = [&](int tn) { return (int64_t)nm * ((ntiles + 4 * tn - 1) / (4 * tn)); };
+  p.tn = 1;
+  if (p.tm == 8) {
+    if (blocks(4) >= cus) p.tn = 4;
+    else if (blocks(2) >= cus) p.tn = 2;
+  }
+  p.slices = 1;
+  static const int kTry[] = {1, 2, 3, 4, 6, 8, 12};
+  for (int s : kTry) {
+    if (ksteps % s || (ksteps / s) % 8) continue;
+    p.slices = s;
+    if (blocks(p.tn) * s * 10 >= cus * 7) break;
+  }
+  return p;
+}
+
+}  // namespace
+
+extern "C" {
+
+int tfd_panel_gemm_slices(int M, int K, int N) {
+  if (M <= 0 || K <= 0 || K % 256 || N <= 0) return 0;
+  return panel_plan(M, K, N).slices;
+}
+
+int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int epilogue,
+                        void* out, void* stream) {
+  if (!x || !w || !out) return fail(kBadArg, "panel_gemm: null pointer");
+  if (M <= 0 || K <= 0 || K % 256 || N <= 0 || N % 4)
+    return fail(kBadShape, "panel_gemm: M=%d K=%d (multiple of 256) N=%d (multiple of 4)", M, K, N);
+  const PanelPlan p = panel_plan(M, K, N);
+  if (epilogue == TFD_PANEL_SWIGLU ? ((N / 2) % 32 || p.slices != 1)
+                                   : epilogue != TFD_PANEL_PARTIAL)
+    return fail(kBadShape, "panel_gemm: epilogue %d with N=%d, %d slices", epilogue, N, p.slices);
+  const int nm = (M + p.tm * 16 - 1) / (p.tm * 16), ntiles = (N + 15) / 16;
+  const int64_t total = (int64_t)nm * ((ntiles + 4 * p.tn - 1) / (4 * p.tn)) * p.slices;
+  const dim3 grid((unsigned)((total + 7) / 8 * 8));
+  const int steps = K / 32 / p.slices;
+  auto s = (hipStream_t)stream;
+#define TFD_PANEL_RUN(TM, TN, KC, DB)                                                           \
+  if (epilogue == TFD_PANEL_SWIGLU)                                                             \
+    hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanSwiglu>), grid, dim3(kBlock), 0, s,   \
+                       (const bf16*)x, (const bf16*)w, M, K, N, p.slices, out);                 \
+  else                                                                                          \
+    hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanPartial>), grid, dim3(kBlock), 0, s,  \
+                       (const bf16*)x, (const bf16*)w, M, K, N, p.slices, out)
+#define TFD_PANEL_DEEP(TM)                                                                      \
+  if (steps % 16 == 0) { TFD_PANEL_RUN(TM, 1, 4, 16); } else { TFD_PANEL_RUN(TM, 1, 4, 8); }
+  if (p.tn == 4) { TFD_PANEL_RUN(8, 4, 2, 2); }
+  else if (p.tn == 2) { TFD_PANEL_RUN(8, 2, 4, 8); }
+  else if (p.tm == 2) { TFD_PANEL_DEEP(2) }
+  else if (p.tm == 4) { TFD_PANEL_DEEP(4) }
+  else if (p.tm == 6) { TFD_PANEL_DEEP(6) }
+  else { TFD_PANEL_DEEP(8) }
+#undef TFD_PANEL_DEEP
+#undef TFD_PANEL_RUN
+  return launched("panel_gemm");
+}
+
+int tfd_panel_swiglu(const float* part, int slices, int M, int N, void* out, void* stream) {
+  if (!part || !out) return fail(kBadArg, "panel_swiglu: null pointer");
+  if (slices <= 0 || M <= 0 || N <= 0 || N % 64)
+    return fail(kBadShape, "panel_swiglu: slices=%d M=%d N=%d", slices, M, N);
+  const int64_t work = (int64_t)M * (N / 4);
+  hipLaunchKernelGGL(k_panel_swiglu, dim3((unsigned)((work + kBlock - 1) / kBlock)), dim3(kBlock),
+                     0, (hipStream_t)stream, part, slices, M, N, (bf16*)out);
+  return launched("panel_swiglu");
+}
+
+int tfd_panel_add_norm(const float* part, int slices, const void* resid, void* h_out,
+                       const void* gamma, void* norm_out, int M, int n, float eps, void* stream) {
+  if ((slices > 0 && !part) || !resid || !gamma || !norm_out)
+    return fail(kBadArg, "panel_add_norm: null pointer");
+  if (slices < 0 || M <= 0 || n <= 0 || n % 32 || n > 8192)
+    return fail(kBadShape, "panel_add_norm: slices=%d M=%d n=%d", slices, M, n);
+  const int per = (n / 8 + kBlock - 1) / kBlock;
+  auto s = (hipStream_t)stream;
+#define TFD_PANEL_NORM(C)                                                                       \
+  hipLaunchKernelGGL((k_panel_add_norm<C>), dim3(M), dim3(kBlock), 0, s, part, slices,          \
+                     (const bf16*)resid, (bf16*)h_out, (const bf16*)gamma, (bf16*)norm_out, M, n, \
+                     eps)
+  if (per == 1) TFD_PANEL_NORM(1);
+  else if (per == 2) TFD_PANEL_NORM(2);
+  else TFD_PANEL_NORM(4);
+#undef TFD_PANEL_NORM
+  return launched("panel_add_norm");
+}
+
+int tfd_panel_qkv_append(const float* part, int slices, int M, int heads, int kv_heads,
+                         int head_dim, const void* gamma_q, const void* gamma_k,
+                         const void* cos_table, const void* sin_table, int rope_rows,
+                         const int32_t* pos, const int32_t* seq, const int32_t* page_table,
+                         int max_pages, void* k_pool, void* v_pool, int num_pages, float scale,
+                         float eps, void* q_out, int32_t* err, void* stream) {
+  if (!part || !gamma_q || !gamma_k || !cos_table || !sin_table || !pos || !seq || !page_table ||
+      !k_pool || !v_pool || !q_out)
+    return fail(kBadArg, "panel_qkv_append: null pointer");
+  if (slices <= 0 || M <= 0 || heads <= 0 || kv_heads <= 0 || heads % kv_heads || max_pages <= 0 ||
+      num_pages <= 0 || (head_dim != 128 && head_dim != 64))
+    return fail(kBadShape, "panel_qkv_append: M=%d heads=%d kv_heads=%d head_dim=%d", M, heads,
+                kv_heads, head_dim);
+  const dim3 grid(M, (heads + 2 * kv_heads + kWavesPerBlock - 1) / kWavesPerBlock);
+  auto s = (hipStream_t)stream;
+#define TFD_PANEL_QKV(D)                                                                        \
+  hipLaunchKernelGGL((k_panel_qkv<D>), grid, dim3(kBlock), 0, s, part, slices, M, heads, kv_heads, \
+                     (const bf16*)gamma_q, (const bf16*)gamma_k, (const bf16*)cos_table,        \
+                     (const bf16*)sin_table, rope_rows, pos, seq, page_table, max_pages,        \
+                     (bf16*)k_pool, (bf16*)v_pool, num_pages, scale, eps, (bf16*)q_out, err)
+  if (head_dim == 128) TFD_PANEL_QKV(128);
+  else TFD_PANEL_QKV(64);
+#undef TFD_PANEL_QKV
+  return launched("panel_qkv_append");
+}
+
+int tfd_panel_attn_rows(int group) { return group > 0 && group <= 8 ? 128 / group : 0; }
+
+int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, int kv_heads,
+                   int head_dim, const int32_t* page_table, int max_pages, const void* k_pool,
+                   const void* v_pool, int num_pages, void* out, int32_t* err, void* stream) {
+  if (!q || !tiles || !page_table || !k_pool || !v_pool || !out)
+    return fail(kBadArg, "panel_attn: null pointer");
+  if (ntiles <= 0 || ntiles > 65535 || heads <= 0 || kv_heads <= 0 || heads % kv_heads ||
+      max_pages <= 0 || num_pages <= 0)
+    return fail(kBadShape, "panel_attn: ntiles=%d heads=%d kv_heads=%d", ntiles, heads, kv_heads);
+  const int G = heads / kv_heads;
+  const dim3 grid(kv_heads, ntiles);
+  auto s = (hipStream_t)stream;
+#define TFD_PANEL_ATTN(D, GG)                                                                   \
+  hipLaunchKernelGGL((k_panel_attn<D, GG>), grid, dim3(kBlock), 0, s, (const bf16*)q,           \
+                     (const PanelTile*)tiles, heads, kv_heads, page_table, max_pages,           \
+                     (const bf16*)k_pool, (const bf16*)v_pool, num_pages, (bf16*)out, err)
+  if (head_dim == 128 && G == 2) TFD_PANEL_ATTN(128, 2);
+  else if (head_dim == 64 && G == 2) TFD_PANEL_ATTN(64, 2);
+  else if (head_dim == 128 && G == 1) TFD_PANEL_ATTN(128, 1);
+  else return fail(kUnsupported, "panel_attn: head_dim=%d group=%d not built", head_dim, G);
+#undef TFD_PANEL_ATTN
+  return launched("panel_attn");
+}
+
+}  // extern "C"

@@ -311,9 +311,8 @@ class BatchEngine:
             from .prefill import Prefill
             self._prefiller = Prefill(self, packed=True)
         self._load_prompts(prompts)
-        for b, p in enumerate(prompts):
-            if len(p) > 1:
-                self._prefiller.run(list(p[:-1]), 0, seq=b)
+        self._prefiller.run_many([(list(p[:-1]), 0, b) for b, p in enumerate(prompts)
+                                  if len(p) > 1])
         self.pos.copy_(torch.tensor([len(p) - 1 for p in prompts], dtype=torch.int32))
         self.ids.copy_(torch.tensor([p[-1] for p in prompts], dtype=torch.int64))
         self._lib.tfd_embed_rows_bf16(ptr(self.w_embed), ptr(self.ids), ptr(self.hid), self.H,

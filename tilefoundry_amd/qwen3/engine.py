@@ -373,8 +373,8 @@ class Engine:
 
     def prefill(self, prompt_ids: list[int]):
         """Load *prompt_ids* and fill the cache of all but its last token in
-        batched passes (``qwen3.prefill``: up to 32 positions per pass through every
-        layer), leaving the engine at the last prompt position: the next decode step
+        batched passes (``qwen3.prefill``: up to 4,096 positions through every layer
+        together), leaving the engine at the last prompt position: the next decode step
         consumes the last prompt token and picks the first new one, exactly where
         walking the prompt step by step would leave it."""
         pl = len(prompt_ids)

@@ -1,31 +1,25 @@
-"""Prompt prefill: up to 32 prompt positions through every layer in one pass.
+"""Prompt prefill: a prompt's positions through every layer together.
 
 The reference's engine walks a prompt one token per replayed decode step
 (``examples/qwen3_1_7b-tilelang/fast/engine.py:261-262``); its placed fixture
 ``tests/fixtures/placed/qwen3_1_7b_pd.py:55-230`` (``layer_prefill``) is the
 batched form: the prompt rows go through the norm, one q/k/v GEMM, q/k norm +
 RoPE, the cache update for every row, causal attention and the MLP GEMMs
-together.  Here a chunk of R <= 32 prompt rows runs each layer as the batched
-decode step does (``batch_engine.py``: MFMA skinny GEMMs, row norms, paged
-attention per (split, kv head, row)), with every row a position of the same
-sequence: row r sits at position c0 + r and all rows share the sequence's page
-table, so row r attends to the cache rows 0 .. c0 + r - 1 the earlier rows
-wrote plus its own key -- the causal attention of the prompt, each position
-valued exactly as a decode step at that position values it (the HIR's rounding
-points; only f32 summation orders differ).
-
-Rows of one chunk append their keys and values to the same cache the later
-rows read, so the scores launch runs twice per layer: the first launch's
-appends (every row's split 0 writes its own position) are complete when the
-second one reads the cache, and the second launch writes the same bits again.
+together.  Here a pass takes up to ``MAX_PASS`` rows, of one or of several
+sequences, through each layer (``csrc/prefill.hip``): every weight is read once per
+pass and every cached key once per 64 rows of a tile, where the decode kernels
+would read them once per 32 rows and once per row.  Each position is valued as a
+decode step at that position values it: the HIR's rounding points, with attention's
+products exact as the XCD kernel takes them, and other f32 summation orders.
 
 Prefill fills the cache for positions start .. start + n - 1 and leaves the
 hidden states of those rows unused: the last prompt token is then decoded as
-before, by the decode step, which produces the first new token.
+before, by the decode step, which produces the first new token.  So the last layer
+stops at its keys and values; nothing reads what would follow.
 
 The same pass serves a batch engine (``batch_engine.py``): its sequences share
-one pool of pages, each with its own page-table row, and a prompt is prefilled
-one sequence at a time through that sequence's row.
+one pool of pages, each with its own page-table row, and the prompts of all of them
+go through together.
 """
 from __future__ import annotations
 
@@ -34,7 +28,7 @@ import torch
 from .. import _lib
 from .._lib import lib, ptr
 
-MAX_ROWS = 32
+MAX_PASS = 4096             # rows of one pass: its workspaces take about 0.3 GB
 
 # The batched attention's grid is (splits, kv heads, rows): about two blocks per
 # compute unit (256 on the MI355X) keeps every split long enough that its tiles
@@ -50,6 +44,38 @@ def attention_splits(rows: int, kv_heads: int, cap: int) -> int:
     return max(1, min(tiles, -(-SPLIT_BLOCKS // (rows * kv_heads))))
 
 
+def plan_passes(segments, max_rows: int, tile_rows: int):
+    """Cut (tokens, start, seq) segments into passes of at most *max_rows* rows ->
+    per pass (ids, pos, seq, tiles): the token, position and sequence of each row, and
+    the attention tiles (first row, rows, sequence, first position), the deepest
+    first (they take longest, so none of them is left to the end of a launch)."""
+    passes, ids, pos, seqs, tiles = [], [], [], [], []
+
+    def close():
+        nonlocal ids, pos, seqs, tiles
+        if ids:
+            tiles.sort(key=lambda t: -(t[3] + t[1]))
+            passes.append((ids, pos, seqs, tiles))
+        ids, pos, seqs, tiles = [], [], [], []
+
+    for tokens, start, seq in segments:
+        done = 0
+        while done < len(tokens):
+            n = min(len(tokens) - done, max_rows - len(ids))
+            if n == 0:
+                close()
+                continue
+            row0, p0 = len(ids), start + done
+            for t in range(0, n, tile_rows):
+                tiles.append((row0 + t, min(tile_rows, n - t), seq, p0 + t))
+            ids.extend(tokens[done:done + n])
+            pos.extend(range(p0, p0 + n))
+            seqs.extend([seq] * n)
+            done += n
+    close()
+    return passes
+
+
 class Prefill:
     """The batched prompt pass over an engine's weights, pools and page table.
 
@@ -58,7 +84,8 @@ class Prefill:
     ([max_pages], or [sequences][max_pages] with ``num_pages`` pages in the
     pool), ``cos``/``sin``, ``cap``).  With *packed* False the projections are
     re-laid once into the skinny GEMMs' operand blocks (one more copy of the
-    layer weights in HBM); a batch engine's layers are already in that order."""
+    layer weights in HBM); a batch engine's layers are already in that order.
+    Workspaces grow to the largest pass seen, ``MAX_PASS`` rows at most."""
 
     def __init__(self, engine, packed: bool = False):
         e = engine
@@ -72,10 +99,8 @@ class Prefill:
         self.eps, self.scale = e.eps, e.scale
         self.max_pages = e.max_pages
         self.num_pages = getattr(e, "num_pages", e.max_pages)
-        self.rows = e.page_table.reshape(-1, self.max_pages)      # [sequences][max_pages]
-        self.nsplit = attention_splits(MAX_ROWS, self.HKV, e.cap)
-        self.split_tiles = 0                  # derived from each row's position
-        self.score_stride = -(-e.cap // _lib.ATTN_SPLIT) * _lib.ATTN_SPLIT
+        self.seqs = e.page_table.numel() // self.max_pages
+        self.tile_rows = self._lib.tfd_panel_attn_rows(self.HQ // self.HKV)
         s = torch.cuda.current_stream(self.dev).cuda_stream
         self.layers = []
         for w in e.layers:
@@ -85,7 +110,7 @@ class Prefill:
                     lw[n] = self._mfma_order(w[n], s)
             self.layers.append(lw)
         torch.cuda.synchronize(self.dev)
-        self._buffers()
+        self.rows = 0
 
     def _mfma_order(self, w, s):
         N, K = w.shape
@@ -93,83 +118,95 @@ class Prefill:
         self._lib.tfd_pack_skinny_bf16(ptr(w), K, N, K, ptr(out), s)
         return out
 
-    def _buffers(self):
-        dev, bf, f32, i32 = self.dev, torch.bfloat16, torch.float32, torch.int32
-        R = MAX_ROWS
+    def _slices(self, M, K, N):
+        return self._lib.tfd_panel_gemm_slices(M, K, N)
 
-        def z(*shape, dtype=bf):
-            return torch.zeros(*shape, device=dev, dtype=dtype)
+    def _reserve(self, M):
+        """Workspaces for passes of up to M rows."""
+        if M <= self.rows:
+            return
+        R = self.rows = -(-M // 32) * 32
+        dev, bf, f32 = self.dev, torch.bfloat16, torch.float32
+        shapes = [(self.H, self.qkv_n), (self.QD, self.H), (self.I, self.H), (self.H, 2 * self.I)]
+        part = 1
+        for K, N in shapes:
+            for m in range(32, R + 1, 32):
+                sl = self._slices(m, K, N)
+                if N != 2 * self.I or sl > 1:      # gate/up: only its K splits leave partials
+                    part = max(part, sl * m * N)
+        self.hid = torch.empty(R, self.H, device=dev, dtype=bf)
+        self.h1 = torch.empty(R, self.H, device=dev, dtype=bf)
+        self.xn = torch.zeros(R * self.H, device=dev, dtype=bf)
+        self.q = torch.empty(R, self.QD, device=dev, dtype=bf)
+        self.attn = torch.zeros(R * self.QD, device=dev, dtype=bf)
+        self.hmid = torch.zeros(R * self.I, device=dev, dtype=bf)
+        self.part = torch.empty(part, device=dev, dtype=f32)
 
-        self.hid = [z(R, self.H), z(R, self.H)]       # ping-pong layer input / output
-        self.xn = z(32 * self.H)
-        self.qkv = z(R, self.qkv_n)
-        self.attn = z(32 * self.QD)
-        self.h1 = z(R, self.H)
-        self.hmid = z(32 * self.I)
-        self.scores = z(R, self.HQ, self.score_stride, dtype=f32)
-        self.smax = z(R, self.nsplit, self.HQ, dtype=f32)
-        self.snew = z(R, self.HQ, dtype=f32)
-        self.psum = z(R, self.nsplit, self.HQ, dtype=f32)
-        self.pout = z(R, self.nsplit, self.HQ, self.D, dtype=f32)
-        self.counters = z(R, self.HKV, dtype=i32)
-        self.pos = z(R, dtype=i32)
-        self.ids = z(R, dtype=torch.int64)
-        self.table = self.rows[:1].expand(R, -1).contiguous()
-        self.work = z(1 << 21, dtype=f32)
+    def _gemm(self, x, w, M, K, N, s):
+        """K-split partial sums of x @ w^T -> their number."""
+        self._lib.tfd_panel_gemm_bf16(ptr(x), ptr(w), M, K, N, _lib.PANEL_PARTIAL, ptr(self.part),
+                                      s)
+        return self._slices(M, K, N)
 
-    def _gemm(self, x, w, R, K, N, epi, resid, out, ldo, s):
-        self._lib.tfd_gemm_skinny_bf16(ptr(x), ptr(w), R, K, N, epi,
-                                       None if resid is None else ptr(resid),
-                                       0 if resid is None else resid.shape[-1], ptr(out), ldo,
-                                       ptr(self.work), self.work.numel(), s)
-
-    def _layer(self, i, R, s):
-        """One decoder layer (model.py:236-266) for R prompt rows."""
+    def _layer(self, i, M, pos, seq, tiles, ntiles, s):
+        """One decoder layer (model.py:236-266) for M prompt rows; xn holds its
+        normalised input.  The last layer stops at its keys and values."""
         L, w, e = self._lib, self.layers[i], self.e
-        H, I, D = self.H, self.I, self.D
-        x_in, x_out = self.hid[i % 2], self.hid[(i + 1) % 2]
-        L.tfd_rmsnorm_rows_bf16(ptr(x_in), H, ptr(w["gamma_in"]), ptr(self.xn), 0, R, H,
-                                self.eps, 1, s)
-        self._gemm(self.xn, w["w_qkv"], R, H, self.qkv_n, _lib.EPI_STORE, None, self.qkv,
-                   self.qkv_n, s)
-        for _ in range(2):      # the first launch's appends complete before the second reads
-            L.tfd_attn_rope_scores_paged_batched(
-                ptr(self.qkv), self.qkv_n, ptr(w["gamma_q"]), ptr(w["gamma_k"]), ptr(e.cos),
-                ptr(e.sin), e.cap, ptr(self.pos), ptr(self.table), self.max_pages,
-                ptr(e.kpool[i]), ptr(e.vpool[i]), self.num_pages, R, self.HQ, self.HKV, D,
-                self.scale, self.eps, ptr(self.scores), self.score_stride, ptr(self.smax),
-                ptr(self.snew), self.nsplit, self.split_tiles, ptr(e.err), s)
-        L.tfd_attn_pv_combine_paged_batched(
-            ptr(self.qkv), self.qkv_n, ptr(self.pos), ptr(self.table), self.max_pages,
-            ptr(e.vpool[i]), self.num_pages, R, self.HQ, self.HKV, D, ptr(self.scores),
-            self.score_stride, ptr(self.smax), ptr(self.snew), ptr(self.psum), ptr(self.pout),
-            self.nsplit, self.split_tiles, ptr(self.counters), ptr(self.attn), ptr(e.err), s)
-        self._gemm(self.attn, w["w_o"], R, self.QD, H, _lib.EPI_RESID, x_in, self.h1, H, s)
-        L.tfd_rmsnorm_rows_bf16(ptr(self.h1), H, ptr(w["gamma_post"]), ptr(self.xn), 0, R, H,
-                                self.eps, 1, s)
-        self._gemm(self.xn, w["w_gu"], R, H, 2 * I, _lib.EPI_SWIGLU, None, self.hmid, 0, s)
-        self._gemm(self.hmid, w["w_down"], R, I, H, _lib.EPI_RESID, self.h1, x_out, H, s)
+        H, I = self.H, self.I
+        table = ptr(e.page_table)
+        sl = self._gemm(self.xn, w["w_qkv"], M, H, self.qkv_n, s)
+        L.tfd_panel_qkv_append(
+            ptr(self.part), sl, M, self.HQ, self.HKV, self.D, ptr(w["gamma_q"]),
+            ptr(w["gamma_k"]), ptr(e.cos), ptr(e.sin), e.cap, pos, seq, table, self.max_pages,
+            ptr(e.kpool[i]), ptr(e.vpool[i]), self.num_pages, self.scale, self.eps, ptr(self.q),
+            ptr(e.err), s)
+        if i + 1 == self.L:
+            return
+        L.tfd_panel_attn(ptr(self.q), tiles, ntiles, self.HQ, self.HKV, self.D, table,
+                         self.max_pages, ptr(e.kpool[i]), ptr(e.vpool[i]), self.num_pages,
+                         ptr(self.attn), ptr(e.err), s)
+        sl = self._gemm(self.attn, w["w_o"], M, self.QD, H, s)
+        L.tfd_panel_add_norm(ptr(self.part), sl, ptr(self.hid), ptr(self.h1),
+                             ptr(w["gamma_post"]), ptr(self.xn), M, H, self.eps, s)
+        if self._slices(M, H, 2 * I) == 1:
+            L.tfd_panel_gemm_bf16(ptr(self.xn), ptr(w["w_gu"]), M, H, 2 * I, _lib.PANEL_SWIGLU,
+                                  ptr(self.hmid), s)
+        else:
+            sl = self._gemm(self.xn, w["w_gu"], M, H, 2 * I, s)
+            L.tfd_panel_swiglu(ptr(self.part), sl, M, 2 * I, ptr(self.hmid), s)
+        sl = self._gemm(self.hmid, w["w_down"], M, I, H, s)
+        L.tfd_panel_add_norm(ptr(self.part), sl, ptr(self.h1), ptr(self.hid),
+                             ptr(self.layers[i + 1]["gamma_in"]), ptr(self.xn), M, H, self.eps, s)
 
     def run(self, tokens: list[int], start: int = 0, seq: int = 0):
         """Fill every layer's cache at positions start .. start + len(tokens) - 1
-        of sequence *seq* (its page-table row) from those tokens (chunks of up to
-        32 rows)."""
+        of sequence *seq* (its page-table row) from those tokens."""
+        self.run_many([(tokens, start, seq)])
+
+    def run_many(self, segments):
+        """``run`` for several (tokens, start, seq) at once; a sequence's segments in
+        the order of their positions."""
         e = self.e
-        if start < 0 or start + len(tokens) > e.cap:
-            raise ValueError(f"prefill: positions {start}..{start + len(tokens) - 1} outside the "
-                             f"cache ({e.cap} positions)")
-        if any(not 0 <= int(t) < e.V for t in tokens):
-            raise ValueError(f"prefill: token ids must lie in [0, {e.V})")
-        if not 0 <= seq < self.rows.shape[0]:
-            raise ValueError(f"prefill: sequence {seq} outside [0, {self.rows.shape[0]})")
-        self.table.copy_(self.rows[seq:seq + 1].expand(MAX_ROWS, -1))
+        for tokens, start, seq in segments:
+            if start < 0 or start + len(tokens) > e.cap:
+                raise ValueError(f"prefill: positions {start}..{start + len(tokens) - 1} outside "
+                                 f"the cache ({e.cap} positions)")
+            if any(not 0 <= int(t) < e.V for t in tokens):
+                raise ValueError(f"prefill: token ids must lie in [0, {e.V})")
+            if not 0 <= seq < self.seqs:
+                raise ValueError(f"prefill: sequence {seq} outside [0, {self.seqs})")
         s = torch.cuda.current_stream(self.dev).cuda_stream
-        for c0 in range(0, len(tokens), MAX_ROWS):
-            chunk = tokens[c0:c0 + MAX_ROWS]
-            R = len(chunk)
-            self.ids[:R].copy_(torch.tensor(chunk, dtype=torch.int64))
-            self.pos[:R].copy_(torch.arange(start + c0, start + c0 + R, dtype=torch.int32))
-            self._lib.tfd_embed_rows_bf16(ptr(e.w_embed), ptr(self.ids), ptr(self.hid[0]),
-                                          self.H, R, self.H, e.V, ptr(e.err), s)
+        for ids, pos, seqs, tiles in plan_passes(segments, MAX_PASS, self.tile_rows):
+            M = len(ids)
+            self._reserve(M)
+            flat = torch.tensor(ids + pos + seqs + [v for t in tiles for v in t],
+                                dtype=torch.int32).to(self.dev)
+            at = ptr(flat)
+            token = flat[:M].to(torch.int64)
+            self._lib.tfd_embed_rows_bf16(ptr(e.w_embed), ptr(token), ptr(self.hid), self.H, M,
+                                          self.H, e.V, ptr(e.err), s)
+            self._lib.tfd_panel_add_norm(None, 0, ptr(self.hid), None,
+                                         ptr(self.layers[0]["gamma_in"]), ptr(self.xn), M, self.H,
+                                         self.eps, s)
             for i in range(self.L):
-                self._layer(i, R, s)
+                self._layer(i, M, at + 4 * M, at + 8 * M, at + 12 * M, len(tiles), s)
