@@ -440,6 +440,133 @@ int tfd_gdn_step_cols(const TfdGdnArgs* args, float* read, int ldr, void* stream
  * groups and partial are not used.  Results equal tfd_moe_experts' bit for bit. */
 int tfd_moe_experts_small(const TfdMoeArgs* args, void* stream);
 
+/* ---- prompt passes of the hybrids ----------------------------------------------
+ * `seqs` sequences, T consecutive tokens of each: row m = b * T + t, M = seqs * T.
+ * Panel order and TFD_PANEL_PARTIAL sums as in tf_decode.h.  The reference walks its
+ * prompts token by token (examples/qwen3_5_35b_a3b-tilelang/run.py,
+ * examples/granite_4_0_h_small-cuda/run.py); each row is valued as a step at its
+ * position values it, f32 summation orders apart. */
+
+/* tfd_panel_gemm_bf16 over tfd_pack_skinny_fp8 weights and their f32 row scales. */
+int tfd_panel_gemm_fp8(const void* x, const void* w, const float* scale, int M, int K, int N,
+                       void* out, void* stream);
+/* out[m][n] = bf16(sum of slices): bf16 rows, or f32 of the bf16 value with f32 != 0.
+ * N % 4 == 0, ldo % 4 == 0. */
+int tfd_panel_sum(const float* part, int slices, int M, int N, void* out, int ldo, int f32,
+                  void* stream);
+/* SwiGLU over the sums of [gate rows | up rows] (N = 2 I), in the policy's rounding ->
+ * panel order [M][I]; I % 32 == 0. */
+int tfd_panel_swiglu_halves(const float* part, int slices, int M, int N, int policy, void* out,
+                            void* stream);
+
+/* The residual stream's update and the next norm, a block per row of n <= 8192 values.
+ * y = bf16(sum of slices of part) [slices 0: no update]; with moe set, y is the experts'
+ * output: routed = sum over k slots of d[m][slot] * weights[m][slot], plus y as the shared
+ * expert's part (times sigmoid(bf16(x_moe[m] . w_shared_scale)) where given), rounded as
+ * tfd_moe_experts rounds.  TFD_POLICY_F32: stream f32 += y; TFD_POLICY_BF16: stream bf16 =
+ * bf16(stream + bf16(y * mult)).  Then, with gamma set, the policy's RMSNorm of the stream
+ * (tfd_rmsnorm_f32_rows / tfd_tf_rmsnorm_rows_bf16) in panel order and / or rows. */
+typedef struct {
+  const float* part;
+  int slices;
+  void* stream_rows;        /* [M][n], in place */
+  float mult;
+  const void* d;            /* bf16 [M][k][n] */
+  const float* weights;     /* [M][k] */
+  const void* x_moe;        /* bf16 [M][n] */
+  const void* w_shared_scale;
+  int moe, k;
+  const void* gamma;
+  void* norm_panels;
+  void* norm_rows;          /* bf16 [M][n] */
+  int M, n, policy;
+  float eps;
+} TfdPanelMixArgs;
+int tfd_panel_mix(const TfdPanelMixArgs* args, void* stream);
+
+/* The routed experts of M rows, grouped by expert in tiles of up to 64 rows: for each
+ * (row, slot) d[row][slot] = the expert's output before its weight, bf16 values.  Weights:
+ * bf16 rows as tfd_moe_experts takes them (fp8 0), or e4m3fn packed as
+ * tfd_moe_experts_packed takes them (fp8 1).  H and I multiples of 128, H <= 8192,
+ * experts <= 256, M * k <= 2^20.  groups: int32
+ * [TFD_PANEL_MOE_WORDS(experts, M * k)]; hidden: bf16 [M * k][I]. */
+#define TFD_PANEL_MOE_WORDS(experts, entries) (4 + 3 * ((experts) + (entries) / 64) + (entries))
+typedef struct {
+  const void* x;            /* bf16 [M][H] */
+  const int32_t* idx;       /* [M][k] */
+  const void *w_gate, *w_up, *w_down;
+  const float *s_gate, *s_up, *s_down;
+  int32_t* groups;
+  void* hidden;
+  void* d;                  /* bf16 [M][k][H] */
+  int M, k, experts, H, I, fp8, policy;
+  int32_t* err;
+} TfdPanelMoeArgs;
+int tfd_panel_moe(const TfdPanelMoeArgs* args, void* stream);
+
+/* A gated-DeltaNet mixer over the rows (tfd_gdn_step for each token in turn): from proj
+ * bf16 [M][ldp] to the out-projection's input in panel order [M][hv * 128].  conv_in /
+ * conv_out and state as tfd_gdn_step's.  Work (f32): qk [2][M][hk * 128], v and read
+ * [M][hv * 128], gates [M][hv][2]. */
+typedef struct {
+  const void* proj;
+  int ldp;
+  const float* conv_in;
+  float* conv_out;
+  float* state;
+  const void *conv_w, *a_log, *dt_bias, *gamma;
+  float *qk, *v, *read, *gates;
+  void* out;
+  int seqs, T, key_heads, value_heads, head_dim;
+  float l2_eps, rms_eps;
+} TfdPanelGdnArgs;
+int tfd_panel_gdn(const TfdPanelGdnArgs* args, void* stream);
+
+/* A Mamba2 mixer over the rows (tfd_mamba_step for each token in turn): from proj bf16
+ * [M][ldp] to the out-projection's input in panel order [M][heads * 64].  Work: x bf16
+ * [M][heads * 64], bc bf16 [M][256], gates f32 [M][heads][2], y bf16 [M][heads * 64]. */
+typedef struct {
+  const void* proj;
+  int ldp;
+  const void* conv_in;
+  void* conv_out;
+  float* state;
+  const void *conv_w, *conv_b, *a_log, *dt_bias, *d_skip, *gamma;
+  void *x, *bc, *y;
+  float* gates;
+  void* out;
+  int seqs, T, heads, head_dim, state_dim;
+  float eps;
+} TfdPanelMambaArgs;
+int tfd_panel_mamba(const TfdPanelMambaArgs* args, void* stream);
+
+/* A hybrid's attention layer over the rows, between its projections: append and causal
+ * attention (tfd_gqa_decode's arithmetic per policy) -> panel order [M][heads * head_dim].
+ * proj bf16 [M][ldp]; tiles as tfd_panel_attn's, of up to TFD_PANEL_GQA_ROWS_* rows.
+ * Work: q (f32 for TFD_POLICY_F32, else bf16) [M][heads * head_dim]; TFD_POLICY_F32: gate
+ * bf16 [M][heads * head_dim], self_scores f32 [M][heads]. */
+#define TFD_PANEL_GQA_ROWS_F32 8
+#define TFD_PANEL_GQA_ROWS_BF16 32
+typedef struct {
+  const void* proj;
+  int ldp;
+  const void *gamma_q, *gamma_k, *cos_table, *sin_table;
+  int rope_rows, rot_dim;
+  const int32_t *pos, *seq, *tiles;
+  int ntiles;
+  const int32_t* page_table;
+  int max_pages;
+  void *k_pool, *v_pool;
+  int num_pages, M, heads, kv_heads, head_dim;
+  float scale, eps;
+  void *q, *gate;
+  float* self_scores;
+  void* out;
+  int policy;
+  int32_t* err;
+} TfdPanelGqaArgs;
+int tfd_panel_gqa(const TfdPanelGqaArgs* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

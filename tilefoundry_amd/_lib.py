@@ -26,6 +26,13 @@ ARGMAX_WORK = 128           # int32 per row of tfd_argmax_rows' two-stage work b
 ATTN_SPLIT = 64
 ROUTE_SOFTMAX_TOPK, ROUTE_TOPK_SOFTMAX = 0, 1
 PANEL_PARTIAL, PANEL_SWIGLU = 0, 1   # tfd_panel_gemm_bf16's outputs
+PANEL_GQA_ROWS_F32, PANEL_GQA_ROWS_BF16 = 8, 32   # rows of a tfd_panel_gqa tile
+
+
+def panel_moe_words(experts: int, entries: int) -> int:
+    """int32 words of tfd_panel_moe's group work buffer (TFD_PANEL_MOE_WORDS)."""
+    return 4 + 3 * (experts + entries // 64) + entries
+
 
 
 def moe_group_words(experts: int, rows: int) -> int:
@@ -120,6 +127,14 @@ SIGNATURES: dict[str, list] = {
     "tfd_rowgemv_bf16": [P, P],
     "tfd_gdn_step_cols": [P, P, I, P],
     "tfd_moe_experts_small": [P, P],
+    "tfd_panel_gemm_fp8": [P, P, P, I, I, I, P, P],
+    "tfd_panel_sum": [P, I, I, I, P, I, I, P],
+    "tfd_panel_swiglu_halves": [P, I, I, I, I, P, P],
+    "tfd_panel_mix": [P, P],
+    "tfd_panel_moe": [P, P],
+    "tfd_panel_gdn": [P, P],
+    "tfd_panel_mamba": [P, P],
+    "tfd_panel_gqa": [P, P],
 }
 RESTYPES = {"tfd_last_error": ctypes.c_char_p, "tfd_sample_work_bytes": ctypes.c_int64}
 UNCHECKED = {"tfd_abi_version", "tfd_decode_persistent_grid", "tfd_panel_gemm_slices",
@@ -260,6 +275,63 @@ class TfdRowGemvArgs(ctypes.Structure):
                 ("gate", c_void_p), ("ldg", c_int), ("head_dim", c_int), ("eps", c_float),
                 ("w", c_void_p), ("K", c_int), ("N", c_int), ("out", c_void_p), ("ldo", c_int),
                 ("epilogue", c_int), ("x_rows", c_void_p), ("ldxr", c_int), ("rows", c_int)]
+
+
+class TfdPanelMixArgs(ctypes.Structure):
+    """``TfdPanelMixArgs`` of include/tf_hybrid.h, field for field."""
+
+    _fields_ = [("part", c_void_p), ("slices", c_int), ("stream_rows", c_void_p),
+                ("mult", c_float),
+                *[(n, c_void_p) for n in ("d", "weights", "x_moe", "w_shared_scale")],
+                ("moe", c_int), ("k", c_int),
+                *[(n, c_void_p) for n in ("gamma", "norm_panels", "norm_rows")],
+                ("M", c_int), ("n", c_int), ("policy", c_int), ("eps", c_float)]
+
+
+class TfdPanelMoeArgs(ctypes.Structure):
+    """``TfdPanelMoeArgs`` of include/tf_hybrid.h, field for field."""
+
+    _fields_ = [*[(n, c_void_p) for n in ("x", "idx", "w_gate", "w_up", "w_down", "s_gate",
+                                           "s_up", "s_down", "groups", "hidden", "d")],
+                *[(n, c_int) for n in ("M", "k", "experts", "H", "I", "fp8", "policy")],
+                ("err", c_void_p)]
+
+
+class TfdPanelGdnArgs(ctypes.Structure):
+    """``TfdPanelGdnArgs`` of include/tf_hybrid.h, field for field."""
+
+    _fields_ = [("proj", c_void_p), ("ldp", c_int),
+                *[(n, c_void_p) for n in ("conv_in", "conv_out", "state", "conv_w", "a_log",
+                                           "dt_bias", "gamma", "qk", "v", "read", "gates",
+                                           "out")],
+                *[(n, c_int) for n in ("seqs", "T", "key_heads", "value_heads", "head_dim")],
+                ("l2_eps", c_float), ("rms_eps", c_float)]
+
+
+class TfdPanelMambaArgs(ctypes.Structure):
+    """``TfdPanelMambaArgs`` of include/tf_hybrid.h, field for field."""
+
+    _fields_ = [("proj", c_void_p), ("ldp", c_int),
+                *[(n, c_void_p) for n in ("conv_in", "conv_out", "state", "conv_w", "conv_b",
+                                           "a_log", "dt_bias", "d_skip", "gamma", "x", "bc", "y",
+                                           "gates", "out")],
+                *[(n, c_int) for n in ("seqs", "T", "heads", "head_dim", "state_dim")],
+                ("eps", c_float)]
+
+
+class TfdPanelGqaArgs(ctypes.Structure):
+    """``TfdPanelGqaArgs`` of include/tf_hybrid.h, field for field."""
+
+    _fields_ = [("proj", c_void_p), ("ldp", c_int),
+                *[(n, c_void_p) for n in ("gamma_q", "gamma_k", "cos_table", "sin_table")],
+                ("rope_rows", c_int), ("rot_dim", c_int),
+                *[(n, c_void_p) for n in ("pos", "seq", "tiles")],
+                ("ntiles", c_int), ("page_table", c_void_p), ("max_pages", c_int),
+                ("k_pool", c_void_p), ("v_pool", c_void_p),
+                *[(n, c_int) for n in ("num_pages", "M", "heads", "kv_heads", "head_dim")],
+                ("scale", c_float), ("eps", c_float),
+                *[(n, c_void_p) for n in ("q", "gate", "self_scores", "out")],
+                ("policy", c_int), ("err", c_void_p)]
 
 
 class TfdDecodeArgs(ctypes.Structure):

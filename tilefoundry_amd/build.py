@@ -21,7 +21,7 @@ ARCH = "gfx950"
 #: dependency of all of them.
 SOURCES = ["qwen3_decode.hip", "qwen3_xcd.hip", "qwen3_batch.hip", "hybrid.hip",
            "gqa_hybrid.hip", "twin_ops.hip", "hybrid_small.hip", "sample.hip",
-           "prefill.hip"]
+           "prefill.hip", "prefill_hybrid.hip"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",

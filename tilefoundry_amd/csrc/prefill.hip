@@ -20,27 +20,32 @@
 #include "host_common.h"
 #include "panel.h"
 #include "tf_decode.h"
+#include "tf_hybrid.h"
 
 using namespace tfd;
 using namespace tfd_host;
 
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-constexpr float kNegInf = -__builtin_huge_valf();
-
-__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                 __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
-// One 16-row x 32-k block of packed weights as a matrix-core operand.
-__device__ __forceinline__ u32x4 weight_block(const bf16* W, int64_t block, int lane) {
-  return load16(W + block * 512 + lane * 8);
-}
+// One 16-row x 32-k block of packed weights: as loaded, and as a matrix-core
+// operand (e4m3fn codes decode exactly to bf16; their row scale multiplies the sum).
+template <bool kFp8>
+struct PanelW {
+  using Raw = u32x4;
+  static __device__ __forceinline__ Raw load(const void* W, int64_t block, int lane) {
+    return load16((const bf16*)W + block * 512 + lane * 8);
+  }
+  static __device__ __forceinline__ u32x4 value(const Raw& r) { return r; }
+};
+template <>
+struct PanelW<true> {
+  using Raw = u32x2;
+  static __device__ __forceinline__ Raw load(const void* W, int64_t block, int lane) {
+    return *(const __attribute__((address_space(1))) u32x2*)((const uint8_t*)W + block * 512 +
+                                                             lane * 8);
+  }
+  static __device__ __forceinline__ u32x4 value(const Raw& r) { return fp8x8_to_bf16(r); }
+};
 
 // ---------------------------------------------------------------------------
 // Y[m][n] = sum_k X[m][k] W[n][k] for M rows in panel order.  A block of four
@@ -67,11 +72,13 @@ __device__ __forceinline__ u32x4 weight_block(const bf16* W, int64_t block, int 
 // ---------------------------------------------------------------------------
 enum PanelEpi { kPanPartial = 0, kPanSwiglu = 1 };
 
-template <int TM, int TN, int KC, int DB, int kEpi>
+template <int TM, int TN, int KC, int DB, int kEpi, bool kFp8 = false>
 __global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__ X,
-                                                        const bf16* __restrict__ W, int M, int K,
+                                                        const void* __restrict__ W, int M, int K,
                                                         int N, int slices,
+                                                        const float* __restrict__ wscale,
                                                         void* __restrict__ out) {
+  using WL = PanelW<kFp8>;
   constexpr int kPasses = KC * TM / 4;       // 16-byte loads per thread of one LDS chunk
   static_assert(DB % KC == 0 && TM % 2 == 0 && KC * TM % 4 == 0, "tile shape");
   __shared__ __align__(16) uint8_t xs[2][KC * TM * 1024];
@@ -106,7 +113,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__
   for (int t = 0; t < TN; ++t)
     wt[t] = (int64_t)min((nb * 4 + wave) * TN + t, ntiles - 1) * ksteps + s0;
 
-  u32x4 xr[kPasses], b[DB][TN];
+  u32x4 xr[kPasses];
+  typename WL::Raw b[DB][TN];
   auto load_x = [&](int step) {
 #pragma unroll
     for (int q = 0; q < kPasses; ++q) xr[q] = load16(xsrc[q] + (int64_t)step * 1024);
@@ -120,7 +128,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__
 #pragma unroll
   for (int u = 0; u < DB; ++u)
 #pragma unroll
-    for (int t = 0; t < TN; ++t) b[u][t] = weight_block(W, wt[t] + u, lane);
+    for (int t = 0; t < TN; ++t) b[u][t] = WL::load(W, wt[t] + u, lane);
   f32x4 c[TM][TN];
 #pragma unroll
   for (int m = 0; m < TM; ++m)
@@ -145,13 +153,15 @@ __global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__
         for (int m = 0; m < TM; ++m)
           a[m] = *reinterpret_cast<const u32x4*>(&xs[cur][(v * TM + m) * 1024 + lane * 16]);
 #pragma unroll
-        for (int t = 0; t < TN; ++t)
+        for (int t = 0; t < TN; ++t) {
+          const u32x4 w = WL::value(b[u][t]);
 #pragma unroll
-          for (int m = 0; m < TM; ++m) c[m][t] = mfma(b[u][t], a[m], c[m][t]);
+          for (int m = 0; m < TM; ++m) c[m][t] = mfma(w, a[m], c[m][t]);
+        }
         if (kMore)
 #pragma unroll
           for (int t = 0; t < TN; ++t)
-            b[u][t] = weight_block(W, wt[t] + k0 + u + DB, lane);
+            b[u][t] = WL::load(W, wt[t] + k0 + u + DB, lane);
         __builtin_amdgcn_sched_barrier(0);
       }
       if (next) {
@@ -179,17 +189,12 @@ __global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__
         *reinterpret_cast<uint32_t*>((bf16*)out + panel_off(row, n / 2, N / 2)) =
             pack2(rbf(silu_f(g0)) * u0, rbf(silu_f(g1)) * u1);
       } else {
-        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)slice * M + row) * N + n) = c[m][t];
+        f32x4 y = c[m][t];
+        if (kFp8) y *= *reinterpret_cast<const f32x4*>(wscale + n);
+        *reinterpret_cast<f32x4*>((float*)out + ((int64_t)slice * M + row) * N + n) = y;
       }
     }
   }
-}
-
-// The sum of a value's K slices, in slice order, rounded once.
-__device__ __forceinline__ float slice_sum(const float* p, int64_t stride, int slices) {
-  float a = p[0];
-  for (int s = 1; s < slices; ++s) a += p[s * stride];
-  return rbf(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -255,6 +260,104 @@ __global__ __launch_bounds__(kBlock) void k_panel_qkv(
 }
 
 // ---------------------------------------------------------------------------
+// The hybrids' attention layers before their scores.  Granite (granite model.py:
+// 310-340): queries, keys and values as projected.  Qwen3.5 (torch_ref.py:335-395):
+// per-head RMSNorm and rotate-half RoPE on the first `rot` dims in f32, the queries
+// scaled; the row's own score q . k of its unrounded key; the output gates apart.
+// A block per (row, kv head).
+// ---------------------------------------------------------------------------
+template <int D, int G, bool kF32>
+__global__ __launch_bounds__(kBlock) void k_panel_gqa_append(
+    const bf16* __restrict__ proj, int ldp, int heads, int kv_heads, const bf16* __restrict__ gq,
+    const bf16* __restrict__ gk, const bf16* __restrict__ cos_t, const bf16* __restrict__ sin_t,
+    int rope_rows, int rot, const int* __restrict__ pos, const int* __restrict__ seq,
+    const int* __restrict__ page_table, int max_pages, bf16* __restrict__ kpool,
+    bf16* __restrict__ vpool, int num_pages, float scale, float eps, void* __restrict__ q_out,
+    bf16* __restrict__ gate_out, float* __restrict__ self_s, int* err) {
+  constexpr int kPer = D / kWave;
+  __shared__ float x_s[G + 1][D];
+  const int m = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const int P = pos[m];
+  if (P < 0 || P >= max_pages * kPage || (kF32 && P >= rope_rows)) {
+    if (tid == 0) raise_error(err, kErrPosRange);
+    return;
+  }
+  const int page = page_table[(int64_t)seq[m] * max_pages + P / kPage];
+  const bool page_ok = page >= 0 && page < num_pages;
+  if (!page_ok && tid == 0) raise_error(err, kErrPageRange);
+  const bf16* row = proj + (int64_t)m * ldp;
+  const int qw = kF32 ? 2 * D : D;           // a query head, and its gate
+  const bf16* krow = row + (int64_t)heads * qw + h * D;
+  const bf16* vrow = krow + (int64_t)kv_heads * D;
+  const int64_t at = (((int64_t)(page_ok ? page : 0) * kv_heads + h) * kPage + P % kPage) * D;
+  if (!kF32) {
+    for (int i = tid; i < G * D / 8; i += kBlock)
+      *reinterpret_cast<u32x4*>((bf16*)q_out + ((int64_t)m * heads + h * G) * D + i * 8) =
+          load16(row + (int64_t)h * G * D + i * 8);
+    if (page_ok && tid < D / 8) {
+      *reinterpret_cast<u32x4*>(kpool + at + tid * 8) = load16(krow + tid * 8);
+      *reinterpret_cast<u32x4*>(vpool + at + tid * 8) = load16(vrow + tid * 8);
+    }
+    return;
+  }
+  for (int r = wave; r < G + 1; r += kWavesPerBlock) {
+    const bf16* src = r < G ? row + (int64_t)(h * G + r) * qw : krow;
+    const bf16* gam = r < G ? gq : gk;
+    float x[kPer], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      x[i] = bf2f(src[lane + kWave * i]);
+      ss += x[i] * x[i];
+    }
+    ss = wave_sum(ss);
+    const float rs = rsqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      x_s[r][lane + kWave * i] = x[i] * rs * bf2f(gam[lane + kWave * i]);
+  }
+  __syncthreads();
+  const bf16* cs = cos_t + (int64_t)P * rot;
+  const bf16* sn = sin_t + (int64_t)P * rot;
+  float kv[kPer], y[kPer];
+  auto rope = [&](int r, float (&o)[kPer]) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int d = lane + kWave * i;
+      const float v = x_s[r][d];
+      if (d < rot) {
+        const float partner = d < rot / 2 ? -x_s[r][d + rot / 2] : x_s[r][d - rot / 2];
+        o[i] = v * bf2f(cs[d]) + partner * bf2f(sn[d]);
+      } else {
+        o[i] = v;
+      }
+    }
+  };
+  rope(G, kv);
+  if (wave == 0 && page_ok) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      kpool[at + lane + kWave * i] = f2bf(kv[i]);
+      vpool[at + lane + kWave * i] = vrow[lane + kWave * i];
+    }
+  }
+  for (int r = wave; r < G; r += kWavesPerBlock) {
+    rope(r, y);
+    const int64_t qh = (int64_t)m * heads + h * G + r;
+    float a = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      y[i] *= scale;
+      a += y[i] * kv[i];
+      ((float*)q_out)[qh * D + lane + kWave * i] = y[i];
+      gate_out[qh * D + lane + kWave * i] = row[(int64_t)(h * G + r) * qw + D + lane + kWave * i];
+    }
+    a = wave_sum(a);
+    if (lane == 0) self_s[qh] = a;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Causal attention of a prompt pass (model.py:190-212) over the paged cache,
 // which already holds the pass's own keys and values.
 //
@@ -280,17 +383,41 @@ struct PanelTile {
   int row0, rows, seq, pos0;
 };
 
-template <int D, int G>
+// Eight f32 values as three bf16 operands: each takes the next eight bits.
+__device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, u32x4 (&o)[3]) {
+  float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    o[i] = u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] -= rbf(v[e]);
+  }
+}
+
+// kPol: the models' arithmetics.  kAttnDense as above.  kAttnGranite: s = bf16(q . k)
+// times the scale in f32, p = bf16(exp(s - m)) with its sum in f32 (granite
+// model.py:310-366; the cache holds the row's own key exactly).  kAttnF32 (Qwen3.5):
+// f32 queries, scores and probabilities; a matrix-core operand is 8 bits wide, so a
+// query and a probability are each three operands whose sum is the f32 value to its
+// last bit, and the row's own score (of its unrounded key) comes from `self_s`; the
+// output is gated by sigmoid(gate).  CT: 16-column tiles per wave.
+enum PanelAttnPolicy { kAttnDense = 0, kAttnGranite = 1, kAttnF32 = 2 };
+
+template <int D, int G, int CT, int kPol>
 __global__ __launch_bounds__(kBlock) void k_panel_attn(
-    const bf16* __restrict__ q, const PanelTile* __restrict__ tiles, int heads, int kv_heads,
+    const void* __restrict__ q_in, const PanelTile* __restrict__ tiles, int heads, int kv_heads,
     const int* __restrict__ page_table, int max_pages, const bf16* __restrict__ kpool,
-    const bf16* __restrict__ vpool, int num_pages, bf16* __restrict__ out, int* err) {
-  constexpr int QT = 128 / G;                // rows of a tile
+    const bf16* __restrict__ vpool, int num_pages, float scale,
+    const float* __restrict__ self_s, const bf16* __restrict__ gate, bf16* __restrict__ out,
+    int* err) {
+  constexpr int QT = 64 * CT / G;            // rows of a tile
+  constexpr int kQ = kPol == kAttnF32 ? 3 : 1;   // operands per query / probability
   constexpr int DS = D / 32, DT = D / 16;    // k steps of q.k, 16-row tiles of V^T
   constexpr int KS = D + 8, VS = 64 + 8;     // LDS row strides (bf16)
   constexpr int kCh = D / 8;                 // 16-byte chunks of a head row
   constexpr int kKPass = 64 * kCh / kBlock;  // K loads per thread and tile
-  constexpr int kVThr = 16 * kCh;            // threads that move V: 4 positions x 8 dims each
+  constexpr int kVThr = 16 * kCh;            // pieces of V: 4 positions x 8 dims each
+  constexpr int kVPass = kVThr > kBlock ? kVThr / kBlock : 1;
   __shared__ __align__(16) bf16 ks[64 * KS];
   __shared__ __align__(16) bf16 vt[D * VS];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
@@ -311,21 +438,31 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
     return 0;
   };
 
-  // this wave's columns: c = 32 wave + 16 ct + r -> query head c / QT, row c % QT
-  u32x4 qf[2][DS];
-  int qpos[2];
+  // this wave's columns: c = 16 (CT wave + ct) + r -> query head c / QT, row c % QT
+  u32x4 qf[CT][DS][kQ];
+  int qpos[CT];
+  float own[CT];
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int c = 32 * wave + 16 * ct + r;
+  for (int ct = 0; ct < CT; ++ct) {
+    const int c = 16 * (CT * wave + ct) + r;
     const int row = min(c % QT, tl.rows - 1);
     qpos[ct] = tl.pos0 + row;
-    const bf16* qp = q + ((int64_t)(tl.row0 + row) * heads + h * G + c / QT) * D;
+    const int64_t qh = (int64_t)(tl.row0 + row) * heads + h * G + c / QT;
+    own[ct] = kPol == kAttnF32 ? self_s[qh] : 0.f;
 #pragma unroll
-    for (int s = 0; s < DS; ++s) qf[ct][s] = load16(qp + 32 * s + 8 * kq);
+    for (int s = 0; s < DS; ++s) {
+      const int64_t at = qh * D + 32 * s + 8 * kq;
+      if constexpr (kPol == kAttnF32) {
+        const f32x4* qp = reinterpret_cast<const f32x4*>((const float*)q_in + at);
+        split3(qp[0], qp[1], qf[ct][s]);
+      } else {
+        qf[ct][s][0] = load16((const bf16*)q_in + at);
+      }
+    }
   }
 
-  u32x4 kr[kKPass], vr[4];
-  const int vg = tid / kCh, vc = tid % kCh;  // V: position group of 4, 8-dim chunk
+  u32x4 kr[kKPass], vr[kVPass][4];
+  const int vc = tid % kCh;                  // V: 8-dim chunk; position group tid / kCh + ..
   auto load_tile = [&](int j0) {
 #pragma unroll
     for (int i = 0; i < kKPass; ++i) {
@@ -333,12 +470,15 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
       kr[i] = load16(kpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
                      (c % kCh) * 8);
     }
-    if (kVThr == kBlock || tid < kVThr) {
-      const int p = j0 + 4 * vg;
-      const bf16* v0 = vpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
-                       vc * 8;
+    if (kVThr >= kBlock || tid < kVThr) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) vr[i] = load16(v0 + i * D);
+      for (int g = 0; g < kVPass; ++g) {
+        const int p = j0 + 4 * ((tid + g * kBlock) / kCh);
+        const bf16* v0 = vpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
+                         vc * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vr[g][i] = load16(v0 + i * D);
+      }
     }
   };
   auto stage_tile = [&]() {
@@ -347,65 +487,84 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
       const int c = tid + i * kBlock;
       *reinterpret_cast<u32x4*>(&ks[(c / kCh) * KS + (c % kCh) * 8]) = kr[i];
     }
-    if (kVThr == kBlock || tid < kVThr) {
+    if (kVThr >= kBlock || tid < kVThr) {
       // positions in the order the probabilities come in: within 32, position
       // 16 t + 4 g + e sits at 8 g + 4 t + e
-      const int at = 32 * (vg >> 3) + 8 * (vg & 3) + 4 * ((vg >> 2) & 1);
 #pragma unroll
-      for (int d = 0; d < 8; ++d) {
-        const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
-        const uint32_t w0 = (d >> 1) == 0 ? vr[0].x : (d >> 1) == 1 ? vr[0].y : (d >> 1) == 2 ? vr[0].z : vr[0].w;
-        const uint32_t w1 = (d >> 1) == 0 ? vr[1].x : (d >> 1) == 1 ? vr[1].y : (d >> 1) == 2 ? vr[1].z : vr[1].w;
-        const uint32_t w2 = (d >> 1) == 0 ? vr[2].x : (d >> 1) == 1 ? vr[2].y : (d >> 1) == 2 ? vr[2].z : vr[2].w;
-        const uint32_t w3 = (d >> 1) == 0 ? vr[3].x : (d >> 1) == 1 ? vr[3].y : (d >> 1) == 2 ? vr[3].z : vr[3].w;
-        const u32x2 o = {__builtin_amdgcn_perm(w1, w0, sel), __builtin_amdgcn_perm(w3, w2, sel)};
-        *reinterpret_cast<u32x2*>(&vt[(vc * 8 + d) * VS + at]) = o;
+      for (int g = 0; g < kVPass; ++g) {
+        const int vg = (tid + g * kBlock) / kCh;
+        const int at = 32 * (vg >> 3) + 8 * (vg & 3) + 4 * ((vg >> 2) & 1);
+        auto word = [&](int i, int d) {
+          const u32x4 v = vr[g][i];
+          return (d >> 1) == 0 ? v.x : (d >> 1) == 1 ? v.y : (d >> 1) == 2 ? v.z : v.w;
+        };
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+          const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
+          *reinterpret_cast<u32x2*>(&vt[(vc * 8 + d) * VS + at]) =
+              u32x2{__builtin_amdgcn_perm(word(1, d), word(0, d), sel),
+                    __builtin_amdgcn_perm(word(3, d), word(2, d), sel)};
+        }
       }
     }
   };
 
-  f32x4 o[DT][2];
-  float mx[2] = {kNegInf, kNegInf}, sum[2] = {0.f, 0.f}, self[2] = {kNegInf, kNegInf};
+  f32x4 o[DT][CT];
+  float mx[CT], sum[CT], self[CT];
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt][0] = o[dt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ct = 0; ct < CT; ++ct) {
+    mx[ct] = self[ct] = kPanelNegInf;
+    sum[ct] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[dt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   load_tile(0);
   for (int j0 = 0; j0 <= last; j0 += 64) {
     stage_tile();
     __syncthreads();
     if (j0 + 64 <= last) load_tile(j0 + 64);
-    f32x4 st[4][2];
+    f32x4 st[4][CT];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) st[p][0] = st[p][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) st[p][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < DS; ++s)
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const u32x4 kf = *reinterpret_cast<const u32x4*>(&ks[(16 * p + r) * KS + 32 * s + 8 * kq]);
-        st[p][0] = mfma(kf, qf[0][s], st[p][0]);
-        st[p][1] = mfma(kf, qf[1][s], st[p][1]);
-      }
-    u32x4 pb[2][2];                          // the packed probabilities of 32 positions each
 #pragma unroll
-    for (int ct = 0; ct < 2; ++ct) {
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int i = kQ - 1; i >= 0; --i) st[p][ct] = mfma(kf, qf[ct][s][i], st[p][ct]);
+      }
+    u32x4 pb[2][CT][kQ];                     // the packed probabilities of 32 positions each
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
       const int before = qpos[ct] - j0 - 4 * kq;   // position 16 p + e is past: 16 p + e < before
-      float tm = kNegInf;
+      float tm = kPanelNegInf;
+      auto score = [&](float v) {
+        return kPol == kAttnDense ? rbf(v) : kPol == kAttnGranite ? rbf(v) * scale : v;
+      };
       if (j0 + 64 > tl.pos0) {               // a tile that reaches the diagonal
 #pragma unroll
         for (int p = 0; p < 4; ++p)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float s = rbf(st[p][ct][e]);
+            float s = score(st[p][ct][e]);
+            if (kPol == kAttnF32 && 16 * p + e == before) s = own[ct];
             if (16 * p + e == before) self[ct] = s;
             if (16 * p + e <= before) tm = fmaxf(tm, s);
-            st[p][ct][e] = 16 * p + e < before ? s : kNegInf;
+            // dense: the own key is a term of its own, added at the end
+            st[p][ct][e] = 16 * p + e < before + (kPol == kAttnDense ? 0 : 1) ? s : kPanelNegInf;
           }
       } else {
 #pragma unroll
         for (int p = 0; p < 4; ++p)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            st[p][ct][e] = rbf(st[p][ct][e]);
+            st[p][ct][e] = score(st[p][ct][e]);
             tm = fmaxf(tm, st[p][ct][e]);
           }
       }
@@ -423,21 +582,22 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
 #pragma unroll
         for (int e = 0; e < 4; ++e) o[dt][ct][e] *= alpha;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        float pe[4];
+      for (int kk = 0; kk < 2; ++kk) {
+        f32x4 pe[2];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          pe[e] = rbf(expf(rbf(st[p][ct][e] - m1)));
-          sum[ct] += pe[e];
-        }
-        const uint32_t w0 = pack2(pe[0], pe[1]), w1 = pack2(pe[2], pe[3]);
-        if (p & 1) {
-          pb[p >> 1][ct].z = w0;
-          pb[p >> 1][ct].w = w1;
-        } else {
-          pb[p >> 1][ct].x = w0;
-          pb[p >> 1][ct].y = w1;
-        }
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float x = st[2 * kk + p][ct][e] - m1;
+            const float v = kPol == kAttnDense ? rbf(expf(rbf(x))) : expf(x);
+            sum[ct] += v;
+            pe[p][e] = v;
+          }
+        if constexpr (kPol == kAttnF32)
+          split3(pe[0], pe[1], pb[kk][ct]);
+        else
+          pb[kk][ct][0] = u32x4{pack2(pe[0].x, pe[0].y), pack2(pe[0].z, pe[0].w),
+                                pack2(pe[1].x, pe[1].y), pack2(pe[1].z, pe[1].w)};
       }
     }
 #pragma unroll
@@ -445,15 +605,17 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const u32x4 vf = *reinterpret_cast<const u32x4*>(&vt[(16 * dt + r) * VS + 32 * kk + 8 * kq]);
-        o[dt][0] = mfma(vf, pb[kk][0], o[dt][0]);
-        o[dt][1] = mfma(vf, pb[kk][1], o[dt][1]);
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int i = kQ - 1; i >= 0; --i) o[dt][ct] = mfma(vf, pb[kk][ct][i], o[dt][ct]);
       }
     __syncthreads();
   }
 
 #pragma unroll
-  for (int ct = 0; ct < 2; ++ct) {
-    const int c = 32 * wave + 16 * ct + r;
+  for (int ct = 0; ct < CT; ++ct) {
+    const int c = 16 * (CT * wave + ct) + r;
     float lo, hi, l = sum[ct], sn = self[ct];
     pair16(l, lo, hi);
     l = lo + hi;
@@ -464,21 +626,33 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
     pair32(sn, lo, hi);
     sn = fmaxf(lo, hi);
     const float pn = rbf(expf(rbf(sn - mx[ct])));
-    const float total = rbf(rbf(l) + pn);
+    const float total = kPol == kAttnDense ? rbf(rbf(l) + pn) : l;
     const int P = qpos[ct];
     const bf16* vrow = vpool + (((int64_t)page_of(P) * kv_heads + h) * kPage + P % kPage) * D;
     const int row = c % QT;
     const int64_t m = tl.row0 + row;
     const int k0 = (h * G + c / QT) * D;
+    const bool on = row < tl.rows;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      const u32x2 vw = *reinterpret_cast<const u32x2*>(vrow + 16 * dt + 4 * kq);
-      const float vn[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
       float y[4];
+      if constexpr (kPol == kAttnDense) {
+        const u32x2 vw = *reinterpret_cast<const u32x2*>(vrow + 16 * dt + 4 * kq);
+        const float vn[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        y[e] = rbf(rbf(o[dt][ct][e]) + rbf(pn * vn[e])) / total;
-      if (row < tl.rows)
+        for (int e = 0; e < 4; ++e) y[e] = rbf(rbf(o[dt][ct][e]) + rbf(pn * vn[e])) / total;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o[dt][ct][e] / total;
+      }
+      if constexpr (kPol == kAttnF32) {
+        const u32x2 gw = *reinterpret_cast<const u32x2*>(
+            gate + (int64_t)(on ? m : tl.row0) * heads * D + k0 + 16 * dt + 4 * kq);
+        const float gn[4] = {bf_lo(gw.x), bf_hi(gw.x), bf_lo(gw.y), bf_hi(gw.y)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] *= 1.f / (1.f + expf(-gn[e]));
+      }
+      if (on)
         *reinterpret_cast<u32x2*>(out + panel_off(m, k0 + 16 * dt + 4 * kq, heads * D)) =
             u32x2{pack2(y[0], y[1]), pack2(y[2], y[3])};
     }
@@ -598,8 +772,8 @@ int tfd_panel_gemm_slices(int M, int K, int N) {
   return panel_plan(M, K, N).slices;
 }
 
-int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int epilogue,
-                        void* out, void* stream) {
+static int panel_gemm(const void* x, const void* w, const float* wscale, int M, int K, int N,
+                      int epilogue, void* out, void* stream) {
   if (!x || !w || !out) return fail(kBadArg, "panel_gemm: null pointer");
   if (M <= 0 || K <= 0 || K % 256 || N <= 0 || N % 4)
     return fail(kBadShape, "panel_gemm: M=%d K=%d (multiple of 256) N=%d (multiple of 4)", M, K, N);
@@ -613,12 +787,15 @@ int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int e
   const int steps = K / 32 / p.slices;
   auto s = (hipStream_t)stream;
 #define TFD_PANEL_RUN(TM, TN, KC, DB)                                                           \
-  if (epilogue == TFD_PANEL_SWIGLU)                                                             \
+  if (wscale)                                                                                   \
+    hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanPartial, true>), grid, dim3(kBlock),  \
+                       0, s, (const bf16*)x, w, M, K, N, p.slices, wscale, out);                \
+  else if (epilogue == TFD_PANEL_SWIGLU)                                                        \
     hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanSwiglu>), grid, dim3(kBlock), 0, s,   \
-                       (const bf16*)x, (const bf16*)w, M, K, N, p.slices, out);                 \
+                       (const bf16*)x, w, M, K, N, p.slices, nullptr, out);                     \
   else                                                                                          \
     hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanPartial>), grid, dim3(kBlock), 0, s,  \
-                       (const bf16*)x, (const bf16*)w, M, K, N, p.slices, out)
+                       (const bf16*)x, w, M, K, N, p.slices, nullptr, out)
 #define TFD_PANEL_DEEP(TM)                                                                      \
   if (steps % 16 == 0) { TFD_PANEL_RUN(TM, 1, 4, 16); } else { TFD_PANEL_RUN(TM, 1, 4, 8); }
   if (p.tn == 4) { TFD_PANEL_RUN(8, 4, 2, 2); }
@@ -630,6 +807,17 @@ int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int e
 #undef TFD_PANEL_DEEP
 #undef TFD_PANEL_RUN
   return launched("panel_gemm");
+}
+
+int tfd_panel_gemm_bf16(const void* x, const void* w, int M, int K, int N, int epilogue,
+                        void* out, void* stream) {
+  return panel_gemm(x, w, nullptr, M, K, N, epilogue, out, stream);
+}
+
+int tfd_panel_gemm_fp8(const void* x, const void* w, const float* scale, int M, int K, int N,
+                       void* out, void* stream) {
+  if (!scale) return fail(kBadArg, "panel_gemm_fp8: null scale");
+  return panel_gemm(x, w, scale, M, K, N, TFD_PANEL_PARTIAL, out, stream);
 }
 
 int tfd_panel_swiglu(const float* part, int slices, int M, int N, void* out, void* stream) {
@@ -701,15 +889,55 @@ int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, i
   const dim3 grid(kv_heads, ntiles);
   auto s = (hipStream_t)stream;
 #define TFD_PANEL_ATTN(D, GG)                                                                   \
-  hipLaunchKernelGGL((k_panel_attn<D, GG>), grid, dim3(kBlock), 0, s, (const bf16*)q,           \
+  hipLaunchKernelGGL((k_panel_attn<D, GG, 2, kAttnDense>), grid, dim3(kBlock), 0, s, q,         \
                      (const PanelTile*)tiles, heads, kv_heads, page_table, max_pages,           \
-                     (const bf16*)k_pool, (const bf16*)v_pool, num_pages, (bf16*)out, err)
+                     (const bf16*)k_pool, (const bf16*)v_pool, num_pages, 1.f, nullptr, nullptr, \
+                     (bf16*)out, err)
   if (head_dim == 128 && G == 2) TFD_PANEL_ATTN(128, 2);
   else if (head_dim == 64 && G == 2) TFD_PANEL_ATTN(64, 2);
   else if (head_dim == 128 && G == 1) TFD_PANEL_ATTN(128, 1);
   else return fail(kUnsupported, "panel_attn: head_dim=%d group=%d not built", head_dim, G);
 #undef TFD_PANEL_ATTN
   return launched("panel_attn");
+}
+
+int tfd_panel_gqa(const TfdPanelGqaArgs* args, void* stream) {
+  if (!args) return fail(kBadArg, "panel_gqa: null args");
+  const TfdPanelGqaArgs& t = *args;
+  const bool f32 = t.policy == TFD_POLICY_F32;
+  if (!f32 && t.policy != TFD_POLICY_BF16) return fail(kBadArg, "panel_gqa: policy %d", t.policy);
+  if (!t.proj || !t.pos || !t.seq || !t.tiles || !t.page_table || !t.k_pool || !t.v_pool ||
+      !t.q || !t.out || (f32 && (!t.gamma_q || !t.gamma_k || !t.cos_table || !t.sin_table ||
+                                 !t.gate || !t.self_scores)))
+    return fail(kBadArg, "panel_gqa: null pointer");
+  const int D = t.head_dim, G = t.kv_heads > 0 ? t.heads / t.kv_heads : 0;
+  const int qw = f32 ? 2 * D : D;
+  if (t.M <= 0 || t.ntiles <= 0 || t.ntiles > 65535 || t.kv_heads <= 0 || t.heads % t.kv_heads ||
+      !(f32 ? D == 256 && G == 8 : D == 128 && G == 4) ||
+      t.ldp < t.heads * qw + 2 * t.kv_heads * D || t.ldp % 8 || t.max_pages <= 0 ||
+      t.num_pages <= 0 ||
+      (f32 && (t.rot_dim <= 0 || t.rot_dim % 2 || t.rot_dim > D || t.rope_rows <= 0)))
+    return fail(kBadShape, "panel_gqa: M=%d tiles=%d heads=%d kv_heads=%d head_dim=%d ldp=%d",
+                t.M, t.ntiles, t.heads, t.kv_heads, D, t.ldp);
+  auto s = (hipStream_t)stream;
+#define TFD_PANEL_GQA(DD, GG, CT, F32, POL)                                                     \
+  hipLaunchKernelGGL((k_panel_gqa_append<DD, GG, F32>), dim3(t.M, t.kv_heads), dim3(kBlock), 0, \
+                     s, (const bf16*)t.proj, t.ldp, t.heads, t.kv_heads,                        \
+                     (const bf16*)t.gamma_q, (const bf16*)t.gamma_k, (const bf16*)t.cos_table,  \
+                     (const bf16*)t.sin_table, t.rope_rows, t.rot_dim, t.pos, t.seq,            \
+                     t.page_table, t.max_pages, (bf16*)t.k_pool, (bf16*)t.v_pool, t.num_pages,  \
+                     t.scale, t.eps, t.q, (bf16*)t.gate, t.self_scores, t.err);                 \
+  hipLaunchKernelGGL((k_panel_attn<DD, GG, CT, POL>), dim3(t.kv_heads, t.ntiles), dim3(kBlock), \
+                     0, s, t.q, (const PanelTile*)t.tiles, t.heads, t.kv_heads, t.page_table,   \
+                     t.max_pages, (const bf16*)t.k_pool, (const bf16*)t.v_pool, t.num_pages,    \
+                     t.scale, t.self_scores, (const bf16*)t.gate, (bf16*)t.out, t.err)
+  if (f32) {
+    TFD_PANEL_GQA(256, 8, 1, true, kAttnF32);
+  } else {
+    TFD_PANEL_GQA(128, 4, 2, false, kAttnGranite);
+  }
+#undef TFD_PANEL_GQA
+  return launched("panel_gqa");
 }
 
 }  // extern "C"

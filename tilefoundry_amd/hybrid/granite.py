@@ -33,6 +33,7 @@ import torch
 from .. import _lib
 from .._lib import lib, ptr
 from ..sampling import Picker, Sampling
+from .prefill import GranitePass, prefill
 from .qwen3_5 import attention_splits, ctypes_addr
 
 BF = torch.bfloat16
@@ -491,22 +492,12 @@ class GraniteEngine:
                                       ptr(self.err), self._stream())
 
     def prefill(self, prompts: list[list[int]]):
-        """Bring every sequence to its prompt's last token: the prompts (all of one
-        length) are walked through the decode step, one position per step, so
-        that the next step decodes each last prompt token.  The recurrent state
-        of the mixers has no batched form here (each position's state is the
-        previous one's update), so this is the walk ``generate`` makes, taken out
-        of it."""
-        if len(prompts) != self.B or any(len(p) < 1 for p in prompts):
-            raise ValueError(f"need {self.B} non-empty prompts")
-        if len({len(p) for p in prompts}) != 1:
-            raise ValueError("prefill: the prompts must have one length (the walk moves "
-                             "every sequence one position per step)")
-        if len(prompts[0]) > self.nsteps:
-            raise ValueError(f"prompt {len(prompts[0])} exceeds {self.nsteps} steps")
-        self._load_prompts(prompts)
-        for _ in range(len(prompts[0]) - 1):
-            self.replay()
+        """Bring every sequence to its prompt's last token (prompts of one length), so
+        that the next step decodes each last prompt token: the positions before it go
+        through the layers in passes of up to 1,024 rows (``hybrid.prefill``), the
+        recurrence alone token by token; sizes those kernels do not take are walked
+        through the decode step, as ``generate`` does."""
+        prefill(self, GranitePass, prompts)
 
     def synthetic_context(self, ctx: int, seed: int = 0):
         """Stand in for a walked `ctx`-token context without walking it: every
