@@ -106,8 +106,12 @@ __device__ __forceinline__ int split_len_of(const GqaArgs& a, int P) {
   return n < kMaxSplitLen ? n : kMaxSplitLen;
 }
 
-// Positions are walked kU passes at a time: every load of the batch is issued
-// before the first is used (positions past the split re-read its last row).
+// Positions are walked kU passes at a time, one batch in use and the next in flight
+// (positions past the split re-read its last row).  The BF16 kernels are bound by the
+// vector units as much as by the cache's stream: a rounded product costs a multiply,
+// half a convert and half a dot (about 20 of the 40 us a kernel takes for 8 Granite rows
+// near 8,190 positions).  With one batch in flight only while nothing is computed, both
+// launches took 83.2 us there, now 76.8; 16 rows near 2,000 positions 55.0 and 48.6.
 constexpr int kU = 4;
 
 // ---------------------------------------------------------------------------
@@ -207,13 +211,14 @@ __global__ __launch_bounds__(kBlock) void k_gqa_scores(GqaArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) qr[g][e] = qk_s[g][li * 8 + e];
   float* srow = a.scores + ((int64_t)b * a.hq + kvh * kG) * a.sstride;
-  for (int jb = 0; jb < n; jb += kPpi * kU) {
-    u32x4 kw[kU];
+  auto load = [&](int jb, u32x4 (&kw)[kU]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int jj = min(jb + u * kPpi + pg, n - 1);
-      kw[u] = load16(a.kpool + page_row(pg_s[jj / kPage], j0 + jj, a.hkv, kvh, kD) + li * 8);
+      kw[u] = load16_stream(a.kpool + page_row(pg_s[jj / kPage], j0 + jj, a.hkv, kvh, kD) + li * 8);
     }
+  };
+  auto use = [&](int jb, const u32x4 (&kw)[kU]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int jj = jb + u * kPpi + pg;
@@ -249,6 +254,17 @@ __global__ __launch_bounds__(kBlock) void k_gqa_scores(GqaArgs a) {
         }
       }
     }
+  };
+  // a batch in use, the next in flight (past the split it re-reads the last row)
+  constexpr int kStep = kPpi * kU;
+  u32x4 ka[kU], kb[kU];
+  load(0, ka);
+  for (int jb = 0; jb < n; jb += 2 * kStep) {
+    load(jb + kStep, kb);
+    use(jb, ka);
+    if (jb + kStep >= n) break;
+    load(jb + 2 * kStep, ka);
+    use(jb + kStep, kb);
   }
   __syncthreads();
   // ---- the split's maximum and sum of exp(x - max), per query head
@@ -311,13 +327,14 @@ __global__ __launch_bounds__(kBlock) void k_gqa_pv(GqaArgs a) {
   for (int g = 0; g < kG; ++g)
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[g][e] = 0.f;
-  for (int jb = 0; jb < n; jb += kPpi * kU) {
-    u32x4 vw[kU];
+  auto load = [&](int jb, u32x4 (&vw)[kU]) {
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const int jj = min(jb + u * kPpi + pg, n - 1);
-      vw[u] = load16(a.vpool + page_row(pg_s[jj / kPage], j0 + jj, a.hkv, kvh, kD) + li * 8);
+      vw[u] = load16_stream(a.vpool + page_row(pg_s[jj / kPage], j0 + jj, a.hkv, kvh, kD) + li * 8);
     }
+  };
+  auto use = [&](int jb, const u32x4 (&vw)[kU]) {
     if constexpr (kF32) {
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
@@ -353,6 +370,16 @@ __global__ __launch_bounds__(kBlock) void k_gqa_pv(GqaArgs a) {
         }
       }
     }
+  };
+  constexpr int kStep = kPpi * kU;
+  u32x4 wa[kU], wb[kU];
+  load(0, wa);
+  for (int jb = 0; jb < n; jb += 2 * kStep) {
+    load(jb + kStep, wb);
+    use(jb, wa);
+    if (jb + kStep >= n) break;
+    load(jb + 2 * kStep, wa);
+    use(jb + kStep, wb);
   }
   // positions of a wave sit kLpp lanes apart; then the waves, in order
 #pragma unroll
