@@ -132,6 +132,11 @@ def test_panel_attn(gpu_device, D, G, segs):
     bf = torch.bfloat16
     k = torch.randn(B * pages, HKV, 16, D, generator=g, device=gpu_device).to(bf)
     v = torch.randn(B * pages, HKV, 16, D, generator=g, device=gpu_device).to(bf)
+    for b, (p0, n) in enumerate(segs):      # what lies past a context is not read
+        at = torch.arange(p0 + n, pages * 16, device=gpu_device)
+        rows = table[b].long()[at // 16]
+        k[rows, :, at % 16] = float("nan")
+        v[rows, :, at % 16] = float("nan")
     M = sum(n for _, n in segs)
     q = (torch.randn(M, heads, D, generator=g, device=gpu_device) * D ** -0.5).to(bf)
     qt = L.tfd_panel_attn_rows(G)

@@ -60,11 +60,13 @@ struct PanelW<true> {
 // SwiGLU's (gate, up) pairs sit in one lane.
 //
 // Bound: at thousands of rows the matrix cores and LDS (a wave reads eight row
-// blocks per 32 matrix products), below 128 rows the weights' stream.  Measured,
-// weights cold (M x K x N): 4,000 x 2048 x 12288 266 us (757 TFLOP/s), 4,000 x 6144 x
-// 2048 117 us (863); 91 x 2048 x 12288 17.8 us (2.8 TB/s of weights); 17 x 2048 x
-// 4096 5.3 us.  The skinny GEMM took 126 launches for the 4,000 rows, 15 us each for
-// 2048 x 12288.
+// blocks per 32 matrix products), below 128 rows the weights' stream and LDS (every
+// row block is read for each column tile).  At four column tiles a wave's registers
+// are held to 256 so that two blocks share a compute unit: with one, 4,000 x 2048 x
+// 12288 took 266 us.  Measured, weights cold (M x K x N): 4,000 x 2048 x 12288 178 us
+// (1,130 TFLOP/s), 4,000 x 6144 x 2048 95 us (1,060); 91 x 2048 x 12288 17.0 us (3.0 TB/s
+// of weights); 17 x 2048 x 4096 5.1 us.  The skinny GEMM took 126 launches for the 4,000
+// rows, 15 us each for 2048 x 12288.
 //
 // grid: 8 x ceil(tiles / 8) blocks.  Consecutive tiles (eight row blocks by a
 // few column blocks) go to one XCD, so that the operands its blocks share stay in
@@ -73,7 +75,7 @@ struct PanelW<true> {
 enum PanelEpi { kPanPartial = 0, kPanSwiglu = 1 };
 
 template <int TM, int TN, int KC, int DB, int kEpi, bool kFp8 = false>
-__global__ __launch_bounds__(kBlock) void k_gemm_panels(const bf16* __restrict__ X,
+__global__ __launch_bounds__(kBlock, 2) void k_gemm_panels(const bf16* __restrict__ X,
                                                         const void* __restrict__ W, int M, int K,
                                                         int N, int slices,
                                                         const float* __restrict__ wscale,
@@ -369,10 +371,14 @@ __global__ __launch_bounds__(kBlock) void k_panel_gqa_append(
 // leave their lane.  K and V tiles are read once per block, prefetched into
 // registers while the tile before is used, V transposed on its way into LDS.
 //
-// Bound: LDS reads and the softmax's VALU work, about equally.  The decode kernels
-// it takes the place of re-read every cached key for each row: a 4,001-token prompt
-// through eight layers took 123.0 ms, with these kernels 7.7 ms; 91 tokens 2.18 and
-// 1.05 ms, eight prompts of 88-700 tokens 51.4 and 5.7 ms (each with one decode step).
+// Bound: the softmax's VALU work (about 1,500 cycles a tile and wave against 1,024 of
+// matrix products and as many of LDS).  4,001 rows take 214 us a layer (302 with a
+// page-table read in front of each load, expf, and an unconditional rescale).
+//
+// The decode kernels it takes the place of re-read every cached key for each row: a
+// 4,001-token prompt through eight layers took 123.0 ms, here 6.02 ms; 91 tokens
+// 2.16 and 1.01 ms, eight prompts of 88-700 tokens 51.4-71 and 5.29 ms (each with
+// one decode step).
 //
 // Rounding: s = bf16(q . k), p = bf16(exp(bf16(s - m))) against the running
 // maximum m (the HIR's final maximum from the tile that holds it on; sums and
@@ -382,6 +388,13 @@ __global__ __launch_bounds__(kBlock) void k_panel_gqa_append(
 struct PanelTile {
   int row0, rows, seq, pos0;
 };
+
+// exp(x) for x <= 0 where the result is rounded to bf16 or summed beside values that
+// are: 2^(x log2 e) on the transcendental unit, off by at most |x| 2^-24 + 2^-22 of the
+// value (below 2^-17 wherever the value is above 2^-40), against 2^-9 of the rounding.
+__device__ __forceinline__ float exp_for_bf16(float x) {
+  return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f);
+}
 
 // Eight f32 values as three bf16 operands: each takes the next eight bits.
 __device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, u32x4 (&o)[3]) {
@@ -404,7 +417,7 @@ __device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, u32x4 (&o
 enum PanelAttnPolicy { kAttnDense = 0, kAttnGranite = 1, kAttnF32 = 2 };
 
 template <int D, int G, int CT, int kPol>
-__global__ __launch_bounds__(kBlock) void k_panel_attn(
+__global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
     const void* __restrict__ q_in, const PanelTile* __restrict__ tiles, int heads, int kv_heads,
     const int* __restrict__ page_table, int max_pages, const bf16* __restrict__ kpool,
     const bf16* __restrict__ vpool, int num_pages, float scale,
@@ -431,11 +444,12 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
     return;
   }
   const int* pt = page_table + (int64_t)tl.seq * max_pages;
-  auto page_of = [&](int p) {                // positions past the pages re-read the last
-    const int pg = pt[min(p, max_pages * kPage - 1) / kPage];
-    if (pg >= 0 && pg < num_pages) return pg;
-    raise_error(err, kErrPageRange);
-    return 0;
+  bool page_bad = false;
+  auto page_at = [&](int i) {                // entries past the table re-read its last
+    const int pg = pt[min(i, max_pages - 1)];
+    const bool ok = pg >= 0 && pg < num_pages;
+    page_bad |= !ok;
+    return ok ? pg : 0;
   };
 
   // this wave's columns: c = 16 (CT wave + ct) + r -> query head c / QT, row c % QT
@@ -463,21 +477,28 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
 
   u32x4 kr[kKPass], vr[kVPass][4];
   const int vc = tid % kCh;                  // V: 8-dim chunk; position group tid / kCh + ..
-  auto load_tile = [&](int j0) {
+  // lane l holds the id of a tile's page l % 4, read a tile ahead of the loads that
+  // need it (a page-table read in front of every load made a tile five round trips)
+  auto load_tile = [&](int j0, int pid) {
 #pragma unroll
     for (int i = 0; i < kKPass; ++i) {
-      const int c = tid + i * kBlock, p = j0 + c / kCh;
-      kr[i] = load16(kpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
+      const int c = tid + i * kBlock, p = c / kCh;
+      const int page = __builtin_amdgcn_readlane(pid, (i * kBlock + wave * kWave) / kCh / kPage);
+      kr[i] = load16(kpool + (((int64_t)page * kv_heads + h) * kPage + p % kPage) * D +
                      (c % kCh) * 8);
     }
     if (kVThr >= kBlock || tid < kVThr) {
 #pragma unroll
       for (int g = 0; g < kVPass; ++g) {
-        const int p = j0 + 4 * ((tid + g * kBlock) / kCh);
-        const bf16* v0 = vpool + (((int64_t)page_of(p) * kv_heads + h) * kPage + p % kPage) * D +
-                         vc * 8;
+        const int at = 4 * ((tid + g * kBlock) / kCh), p = j0 + at;
+        const int page = __shfl(pid, at / kPage, kWave);
+        const bf16* v0 = vpool + (((int64_t)page * kv_heads + h) * kPage + p % kPage) * D + vc * 8;
+        // positions past the last row hold anything (their p is 0): their V reads as 0
 #pragma unroll
-        for (int i = 0; i < 4; ++i) vr[g][i] = load16(v0 + i * D);
+        for (int i = 0; i < 4; ++i) {
+          const u32x4 v = load16(v0 + i * D);
+          vr[g][i] = p + i <= last ? v : u32x4{0u, 0u, 0u, 0u};
+        }
       }
     }
   };
@@ -519,11 +540,19 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
     for (int dt = 0; dt < DT; ++dt) o[dt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  load_tile(0);
+  int pid = page_at(lane & 3);
+  int own_page[CT];
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) own_page[ct] = kPol == kAttnDense ? page_at(qpos[ct] / kPage) : 0;
+  load_tile(0, pid);
+  pid = page_at(4 + (lane & 3));
   for (int j0 = 0; j0 <= last; j0 += 64) {
     stage_tile();
     __syncthreads();
-    if (j0 + 64 <= last) load_tile(j0 + 64);
+    if (j0 + 64 <= last) {
+      load_tile(j0 + 64, pid);
+      pid = page_at(j0 / kPage + 8 + (lane & 3));
+    }
     f32x4 st[4][CT];
 #pragma unroll
     for (int p = 0; p < 4; ++p)
@@ -574,13 +603,16 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
       pair32(tm, lo, hi);
       tm = fmaxf(lo, hi);
       const float m1 = fmaxf(mx[ct], tm);
-      const float alpha = expf(mx[ct] - m1);
-      mx[ct] = m1;
-      sum[ct] *= alpha;
+      // once the tiles that hold the maxima are past, no column's maximum moves
+      if (__any(m1 != mx[ct])) {
+        const float alpha = expf(mx[ct] - m1);
+        mx[ct] = m1;
+        sum[ct] *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[dt][ct][e] *= alpha;
+          for (int e = 0; e < 4; ++e) o[dt][ct][e] *= alpha;
+      }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         f32x4 pe[2];
@@ -589,15 +621,23 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float x = st[2 * kk + p][ct][e] - m1;
-            const float v = kPol == kAttnDense ? rbf(expf(rbf(x))) : expf(x);
-            sum[ct] += v;
-            pe[p][e] = v;
+            pe[p][e] = kPol == kAttnDense ? exp_for_bf16(rbf(x)) :
+                       kPol == kAttnGranite ? exp_for_bf16(x) : expf(x);
+            if (kPol != kAttnDense) sum[ct] += pe[p][e];
           }
-        if constexpr (kPol == kAttnF32)
+        if constexpr (kPol == kAttnF32) {
           split3(pe[0], pe[1], pb[kk][ct]);
-        else
+        } else {
           pb[kk][ct][0] = u32x4{pack2(pe[0].x, pe[0].y), pack2(pe[0].z, pe[0].w),
                                 pack2(pe[1].x, pe[1].y), pack2(pe[1].z, pe[1].w)};
+          if (kPol == kAttnDense) {          // the sum of the rounded probabilities
+            const u32x4 w = pb[kk][ct][0];
+            sum[ct] = dot2(w.x, 0x3f803f80u, sum[ct]);
+            sum[ct] = dot2(w.y, 0x3f803f80u, sum[ct]);
+            sum[ct] = dot2(w.z, 0x3f803f80u, sum[ct]);
+            sum[ct] = dot2(w.w, 0x3f803f80u, sum[ct]);
+          }
+        }
       }
     }
 #pragma unroll
@@ -626,9 +666,9 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
     pair32(sn, lo, hi);
     sn = fmaxf(lo, hi);
     const float pn = rbf(expf(rbf(sn - mx[ct])));
-    const float total = kPol == kAttnDense ? rbf(rbf(l) + pn) : l;
+    const float inv = 1.f / (kPol == kAttnDense ? rbf(rbf(l) + pn) : l);
     const int P = qpos[ct];
-    const bf16* vrow = vpool + (((int64_t)page_of(P) * kv_heads + h) * kPage + P % kPage) * D;
+    const bf16* vrow = vpool + (((int64_t)own_page[ct] * kv_heads + h) * kPage + P % kPage) * D;
     const int row = c % QT;
     const int64_t m = tl.row0 + row;
     const int k0 = (h * G + c / QT) * D;
@@ -640,10 +680,10 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
         const u32x2 vw = *reinterpret_cast<const u32x2*>(vrow + 16 * dt + 4 * kq);
         const float vn[4] = {bf_lo(vw.x), bf_hi(vw.x), bf_lo(vw.y), bf_hi(vw.y)};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = rbf(rbf(o[dt][ct][e]) + rbf(pn * vn[e])) / total;
+        for (int e = 0; e < 4; ++e) y[e] = rbf(rbf(o[dt][ct][e]) + rbf(pn * vn[e])) * inv;
       } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = o[dt][ct][e] / total;
+        for (int e = 0; e < 4; ++e) y[e] = o[dt][ct][e] * inv;
       }
       if constexpr (kPol == kAttnF32) {
         const u32x2 gw = *reinterpret_cast<const u32x2*>(
@@ -657,6 +697,7 @@ __global__ __launch_bounds__(kBlock) void k_panel_attn(
             u32x2{pack2(y[0], y[1]), pack2(y[2], y[3])};
     }
   }
+  if (page_bad) raise_error(err, kErrPageRange);
 }
 
 // ---------------------------------------------------------------------------
@@ -670,12 +711,13 @@ __global__ __launch_bounds__(kBlock) void k_panel_add_norm(
   __shared__ float red[kWavesPerBlock];
   const int64_t m = blockIdx.x;
   const int tid = threadIdx.x, nch = n / 8;
-  u32x4 x[kCh];
+  u32x4 x[kCh], gm[kCh];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < kCh; ++i) {
     const int c = min(tid + i * kBlock, nch - 1);
     const u32x4 rv = load16(resid + m * n + c * 8);
+    gm[i] = load16(gamma + c * 8);
     float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < slices; ++s) {
       const f32x4* p = reinterpret_cast<const f32x4*>(part + ((int64_t)s * M + m) * n + c * 8);
@@ -713,7 +755,7 @@ __global__ __launch_bounds__(kBlock) void k_panel_add_norm(
     const int c = tid + i * kBlock;
     if (c < nch)
       *reinterpret_cast<u32x4*>(norm_out + panel_off(m, c * 8, n)) =
-          rms_norm_chunk(x[i], load16(gamma + c * 8), rs);
+          rms_norm_chunk(x[i], gm[i], rs);
   }
 }
 
@@ -735,8 +777,13 @@ __global__ __launch_bounds__(kBlock) void k_panel_swiglu(const float* __restrict
 
 // ---------------------------------------------------------------------------
 // Tile shape and K slices of a panel GEMM: 16-row tiles per block (every row up
-// to 128, else 128), column tiles per wave, and as few slices as give the chip's
-// compute units a block each.
+// to 128, else 128), column tiles per wave (more of them read LDS less per product;
+// fewer make more blocks), and as few K slices as give most compute units a block --
+// nine tenths of them where K is deep and a block runs long.  Measured (us), the rule's
+// choice against the nearest others: 250 x 2048 x 4096 11.3 (2 tiles, 4 slices), 12.3 (1,
+// 2), 13.5 (2, 2); 250 x 6144 x 2048 13.4 (2, 8), 18.2 (1, 3); 1,000 x 2048 x 12288 58.8
+// (2, 1), 63.0 (4, 1); 1,300 x 2048 x 12288 86.1 (4, 1), 87.3 (2, 1); 4,000 x 2048 x 12288
+// 177.6 (4, 1), 225 (2, 1).
 // ---------------------------------------------------------------------------
 struct PanelPlan {
   int tm, tn, slices;
@@ -748,17 +795,13 @@ PanelPlan panel_plan(int M, int K, int N) {
   p.tm = M <= 128 ? (M + 31) / 32 * 2 : 8;
   const int nm = (M + p.tm * 16 - 1) / (p.tm * 16);
   auto blocks = [&](int tn) { return (int64_t)nm * ((ntiles + 4 * tn - 1) / (4 * tn)); };
-  p.tn = 1;
-  if (p.tm == 8) {
-    if (blocks(4) >= cus) p.tn = 4;
-    else if (blocks(2) >= cus) p.tn = 2;
-  }
+  p.tn = M <= 128 ? 1 : M <= 1024 ? 2 : 4;
   p.slices = 1;
   static const int kTry[] = {1, 2, 3, 4, 6, 8, 12};
   for (int s : kTry) {
     if (ksteps % s || (ksteps / s) % 8) continue;
     p.slices = s;
-    if (blocks(p.tn) * s * 10 >= cus * 7) break;
+    if (blocks(p.tn) * s * 10 >= cus * (K > 4096 ? 9 : 7)) break;
   }
   return p;
 }
@@ -796,14 +839,14 @@ static int panel_gemm(const void* x, const void* w, const float* wscale, int M, 
   else                                                                                          \
     hipLaunchKernelGGL((k_gemm_panels<TM, TN, KC, DB, kPanPartial>), grid, dim3(kBlock), 0, s,  \
                        (const bf16*)x, w, M, K, N, p.slices, nullptr, out)
-#define TFD_PANEL_DEEP(TM)                                                                      \
-  if (steps % 16 == 0) { TFD_PANEL_RUN(TM, 1, 4, 16); } else { TFD_PANEL_RUN(TM, 1, 4, 8); }
+#define TFD_PANEL_DEEP(TM, KC)                                                                  \
+  if (steps % 16 == 0) { TFD_PANEL_RUN(TM, 1, KC, 16); } else { TFD_PANEL_RUN(TM, 1, KC, 8); }
   if (p.tn == 4) { TFD_PANEL_RUN(8, 4, 2, 2); }
   else if (p.tn == 2) { TFD_PANEL_RUN(8, 2, 4, 8); }
-  else if (p.tm == 2) { TFD_PANEL_DEEP(2) }
-  else if (p.tm == 4) { TFD_PANEL_DEEP(4) }
-  else if (p.tm == 6) { TFD_PANEL_DEEP(6) }
-  else { TFD_PANEL_DEEP(8) }
+  else if (p.tm == 2) { TFD_PANEL_DEEP(2, 8) }
+  else if (p.tm == 4) { TFD_PANEL_DEEP(4, 8) }
+  else if (p.tm == 6) { TFD_PANEL_DEEP(6, 8) }
+  else { TFD_PANEL_DEEP(8, 4) }
 #undef TFD_PANEL_DEEP
 #undef TFD_PANEL_RUN
   return launched("panel_gemm");
