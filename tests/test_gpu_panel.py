@@ -28,7 +28,8 @@ def unpanel(flat, M, K):
 def test_plan_passes_covers_every_row_once(lens, max_rows, tile):
     segments = [([1000 * b + i for i in range(n)], 5 * b, b) for b, n in enumerate(lens)]
     seen = []
-    for ids, pos, seqs, tiles in plan_passes(segments, max_rows, tile):
+    for plan in plan_passes(segments, max_rows, tile):
+        ids, pos, seqs, tiles = (a.tolist() for a in plan)
         assert 0 < len(ids) <= max_rows and len(ids) == len(pos) == len(seqs)
         rows = []
         for row0, n, seq, p0 in tiles:
@@ -188,3 +189,23 @@ def test_passes_cut_anywhere_fill_the_same_cache(gpu_device, monkeypatch):
     eng.check_errors()
     assert_close_bf16(eng.kpool, k, max_rel=2e-2, name="k")
     assert_close_bf16(eng.vpool, v, max_rel=2e-2, name="v")
+
+
+def test_token_array_takes_what_a_prompt_may_be():
+    """Lists, tuples, arrays and tensors of ids; what does not fit is refused."""
+    import numpy as np
+
+    from tilefoundry_amd.qwen3.prefill import in_vocab, int32_ids, token_array
+
+    for p in ([1, 2, 3], (1, 2, 3), np.array([1, 2, 3], np.int32), torch.tensor([1, 2, 3]),
+              [torch.tensor(1), 2, np.int64(3)]):
+        assert token_array(p).tolist() == [1, 2, 3] and token_array(p).dtype == np.int64
+    assert token_array([]).size == 0 and in_vocab(token_array([]), 5)
+    assert in_vocab(token_array([0, 4]), 5)
+    assert not in_vocab(token_array([0, 5]), 5) and not in_vocab(token_array([-1]), 5)
+    with pytest.raises(ValueError):
+        token_array([1 << 70])
+    with pytest.raises(ValueError):
+        token_array([[1, 2], [3, 4]])
+    with pytest.raises(RuntimeError):
+        int32_ids([(1 << 32) + 5])

@@ -17,11 +17,12 @@ from __future__ import annotations
 
 import ctypes
 
+import numpy as np
 import torch
 
 from .. import _lib
 from .._lib import lib, ptr
-from ..qwen3.prefill import plan_passes
+from ..qwen3.prefill import plan_passes, token_array
 
 MAX_PASS = 1024             # rows of one pass: its workspaces take up to about 0.4 GB
 
@@ -156,15 +157,16 @@ class _Pass:
         """Positions 0 .. n - 2 of every sequence (prompts of one length n), from the
         engine's state as ``_load_prompts`` leaves it."""
         e, n = self.e, len(prompts[0]) - 1
+        prompts = [token_array(p) for p in prompts]
         span = max(1, MAX_PASS // self.B)
         for t0 in range(0, n, span):
             T = min(span, n - t0)
             M = self.B * T
             self._reserve(M)
-            segments = [(list(p[t0:t0 + T]), t0, b) for b, p in enumerate(prompts)]
+            segments = [(p[t0:t0 + T], t0, b) for b, p in enumerate(prompts)]
             (ids, pos, seqs, tiles), = plan_passes(segments, M, self.tile_rows)
-            flat = torch.tensor(ids + pos + seqs + [v for t in tiles for v in t],
-                                dtype=torch.int32).to(self.dev)
+            flat = torch.from_numpy(np.concatenate((ids, pos, seqs, tiles.reshape(-1)))).to(
+                self.dev)
             token = flat[:M].to(torch.int64)
             s = self._stream()
             self._lib.tfd_embed_rows_bf16(ptr(e.embed), ptr(token), ptr(self.emb), self.H, M,

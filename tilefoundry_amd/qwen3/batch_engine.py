@@ -18,6 +18,7 @@ from __future__ import annotations
 
 from time import perf_counter
 
+import numpy as np
 import torch
 
 from .. import _lib
@@ -25,7 +26,7 @@ from .._lib import lib, ptr
 from ..sampling import Picker, Sampling
 from .config import Qwen3Config
 from .engine import bf16_scale, scatter_cache
-from .prefill import attention_splits
+from .prefill import Prefill, attention_splits, in_vocab, int32_ids, token_array
 from .weights import head_rows, pack_layer, validate
 
 MAX_BATCH = 32
@@ -265,12 +266,13 @@ class BatchEngine:
     def _load_prompts(self, prompts: list[list[int]]):
         self._reset()
         self.inp.zero_()
-        lens = []
+        lens = [len(p) for p in prompts]
+        rows = np.zeros((self.B, max(lens)), dtype=np.int32)
         for b, p in enumerate(prompts):
-            self.inp[b, :len(p)] = torch.tensor(p, dtype=torch.int32).to(self.device)
-            lens.append(len(p))
+            rows[b, :len(p)] = int32_ids(p)
+        self.inp[:, :max(lens)] = torch.from_numpy(rows).to(self.device)
         self.plen.copy_(torch.tensor(lens, dtype=torch.int32))
-        self.ids.copy_(torch.tensor([p[0] for p in prompts], dtype=torch.int64))
+        self.ids.copy_(torch.tensor([int(p[0]) for p in prompts], dtype=torch.int64))
         self._lib.tfd_embed_rows_bf16(ptr(self.w_embed), ptr(self.ids), ptr(self.hid), self.H,
                                       self.B, self.H, self.V, ptr(self.err), self._stream())
 
@@ -308,13 +310,11 @@ class BatchEngine:
         if len(prompts) != self.B or any(len(p) < 1 for p in prompts):
             raise ValueError(f"need {self.B} non-empty prompts")
         if getattr(self, "_prefiller", None) is None:
-            from .prefill import Prefill
             self._prefiller = Prefill(self, packed=True)
         self._load_prompts(prompts)
-        self._prefiller.run_many([(list(p[:-1]), 0, b) for b, p in enumerate(prompts)
-                                  if len(p) > 1])
+        self._prefiller.run_many([(p[:-1], 0, b) for b, p in enumerate(prompts) if len(p) > 1])
         self.pos.copy_(torch.tensor([len(p) - 1 for p in prompts], dtype=torch.int32))
-        self.ids.copy_(torch.tensor([p[-1] for p in prompts], dtype=torch.int64))
+        self.ids.copy_(torch.tensor([int(p[-1]) for p in prompts], dtype=torch.int64))
         self._lib.tfd_embed_rows_bf16(ptr(self.w_embed), ptr(self.ids), ptr(self.hid), self.H,
                                       self.B, self.H, self.V, ptr(self.err), self._stream())
 
@@ -343,7 +343,8 @@ class BatchEngine:
         if longest + max_new > self.nsteps:
             raise ValueError(f"prompt {longest} + {max_new} new exceeds this engine's "
                              f"{self.nsteps} steps")
-        if any(not 0 <= int(t) < self.V for p in prompts for t in p):
+        prompts = [token_array(p) for p in prompts]
+        if not all(in_vocab(p, self.V) for p in prompts):
             raise ValueError(f"prompt ids must lie in [0, {self.V})")
         torch.cuda.synchronize(self.device)
         t_pre = perf_counter()

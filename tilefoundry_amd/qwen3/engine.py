@@ -29,6 +29,7 @@ import torch
 from .. import _lib
 from .._lib import lib, ptr
 from .config import Qwen3Config
+from .prefill import Prefill, in_vocab, int32_ids, token_array
 from .weights import head_rows, pack_layer, validate
 
 
@@ -352,7 +353,7 @@ class Engine:
         pl = len(prompt_ids)
         self._reset()
         self.inp.zero_()
-        self.inp[:pl] = torch.tensor(prompt_ids, dtype=torch.int32).to(self.device)
+        self.inp[:pl] = torch.from_numpy(int32_ids(prompt_ids)).to(self.device)
         self.plen.fill_(pl)
         self.ids.fill_(int(prompt_ids[0]))
         self._embed_current()
@@ -382,9 +383,8 @@ class Engine:
         if pl < 2:
             return
         if getattr(self, "_prefiller", None) is None:
-            from .prefill import Prefill
             self._prefiller = Prefill(self)
-        self._prefiller.run(list(prompt_ids[:-1]), 0)
+        self._prefiller.run(prompt_ids[:-1], 0)
         self.pos.fill_(pl - 1)
         self.ids.fill_(int(prompt_ids[-1]))
         self._embed_current()
@@ -400,7 +400,8 @@ class Engine:
         if pl + max_new > self.nsteps:
             raise ValueError(f"prompt {pl} + {max_new} new exceeds this engine's "
                              f"{self.nsteps} steps")
-        if any(not 0 <= int(t) < self.V for t in prompt_ids):
+        prompt_ids = token_array(prompt_ids)
+        if not in_vocab(prompt_ids, self.V):
             raise ValueError(f"prompt ids must lie in [0, {self.V})")
         hist = (torch.empty(max_new, self.V, device=self.device, dtype=torch.float32)
                 if record_logits else None)

@@ -23,6 +23,7 @@ go through together.
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from .. import _lib
@@ -44,33 +45,65 @@ def attention_splits(rows: int, kv_heads: int, cap: int) -> int:
     return max(1, min(tiles, -(-SPLIT_BLOCKS // (rows * kv_heads))))
 
 
+def token_array(tokens) -> np.ndarray:
+    """Token ids (any sequence of them) as an int64 array."""
+    try:
+        ids = np.asarray(tokens, dtype=np.int64)
+    except TypeError:                       # values numpy cannot read, e.g. on a device
+        ids = np.array([int(t) for t in tokens], dtype=np.int64)
+    except OverflowError:
+        raise ValueError("token ids must fit in 64 bits") from None
+    if ids.ndim != 1:
+        raise ValueError(f"token ids must be one sequence, got {ids.ndim} dimensions")
+    return ids
+
+
+def int32_ids(tokens) -> np.ndarray:
+    """``token_array`` as the int32 values the device buffers hold."""
+    ids = token_array(tokens)
+    if not in_vocab(np.abs(ids), 1 << 31):
+        raise RuntimeError("token ids must fit in 32 bits")
+    return ids.astype(np.int32)
+
+
+def in_vocab(tokens: np.ndarray, vocab: int) -> bool:
+    return tokens.size == 0 or (int(tokens.min()) >= 0 and int(tokens.max()) < vocab)
+
+
 def plan_passes(segments, max_rows: int, tile_rows: int):
     """Cut (tokens, start, seq) segments into passes of at most *max_rows* rows ->
-    per pass (ids, pos, seq, tiles): the token, position and sequence of each row, and
-    the attention tiles (first row, rows, sequence, first position), the deepest
-    first (they take longest, so none of them is left to the end of a launch)."""
-    passes, ids, pos, seqs, tiles = [], [], [], [], []
+    per pass (ids, pos, seq, tiles), int32 arrays: the token, position and sequence of
+    each row, and the attention tiles [n][4] (first row, rows, sequence, first position),
+    the deepest first (they take longest, so none of them is left to the end of a
+    launch)."""
+    passes, parts, rows = [], [], 0
 
     def close():
-        nonlocal ids, pos, seqs, tiles
-        if ids:
-            tiles.sort(key=lambda t: -(t[3] + t[1]))
-            passes.append((ids, pos, seqs, tiles))
-        ids, pos, seqs, tiles = [], [], [], []
+        nonlocal parts, rows
+        if parts:
+            ids = np.concatenate([t for t, _, _ in parts]).astype(np.int32)
+            pos = np.concatenate([np.arange(p, p + len(t), dtype=np.int32) for t, p, _ in parts])
+            seqs = np.concatenate([np.full(len(t), q, dtype=np.int32) for t, _, q in parts])
+            tiles, row0 = [], 0
+            for t, p, q in parts:
+                at = np.arange(0, len(t), tile_rows, dtype=np.int32)
+                tiles.append(np.stack((row0 + at, np.minimum(tile_rows, len(t) - at),
+                                       np.full_like(at, q), p + at), axis=1))
+                row0 += len(t)
+            tiles = np.concatenate(tiles)
+            tiles = tiles[np.argsort(-(tiles[:, 3] + tiles[:, 1]), kind="stable")]
+            passes.append((ids, pos, seqs, tiles.astype(np.int32)))
+        parts, rows = [], 0
 
     for tokens, start, seq in segments:
-        done = 0
+        tokens, done = token_array(tokens), 0
         while done < len(tokens):
-            n = min(len(tokens) - done, max_rows - len(ids))
+            n = min(len(tokens) - done, max_rows - rows)
             if n == 0:
                 close()
                 continue
-            row0, p0 = len(ids), start + done
-            for t in range(0, n, tile_rows):
-                tiles.append((row0 + t, min(tile_rows, n - t), seq, p0 + t))
-            ids.extend(tokens[done:done + n])
-            pos.extend(range(p0, p0 + n))
-            seqs.extend([seq] * n)
+            parts.append((tokens[done:done + n], start + done, seq))
+            rows += n
             done += n
     close()
     return passes
@@ -191,7 +224,7 @@ class Prefill:
             if start < 0 or start + len(tokens) > e.cap:
                 raise ValueError(f"prefill: positions {start}..{start + len(tokens) - 1} outside "
                                  f"the cache ({e.cap} positions)")
-            if any(not 0 <= int(t) < e.V for t in tokens):
+            if not in_vocab(token_array(tokens), e.V):
                 raise ValueError(f"prefill: token ids must lie in [0, {e.V})")
             if not 0 <= seq < self.seqs:
                 raise ValueError(f"prefill: sequence {seq} outside [0, {self.seqs})")
@@ -199,8 +232,8 @@ class Prefill:
         for ids, pos, seqs, tiles in plan_passes(segments, MAX_PASS, self.tile_rows):
             M = len(ids)
             self._reserve(M)
-            flat = torch.tensor(ids + pos + seqs + [v for t in tiles for v in t],
-                                dtype=torch.int32).to(self.dev)
+            flat = torch.from_numpy(np.concatenate((ids, pos, seqs, tiles.reshape(-1)))).to(
+                self.dev)
             at = ptr(flat)
             token = flat[:M].to(torch.int64)
             self._lib.tfd_embed_rows_bf16(ptr(e.w_embed), ptr(token), ptr(self.hid), self.H, M,
