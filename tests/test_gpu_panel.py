@@ -209,3 +209,23 @@ def test_token_array_takes_what_a_prompt_may_be():
         token_array([[1, 2], [3, 4]])
     with pytest.raises(RuntimeError):
         int32_ids([(1 << 32) + 5])
+
+
+@pytest.mark.parametrize("batch", [8, 9, 17, 32])
+def test_batch_step_on_both_sides_of_nine_rows(gpu_device, batch):
+    """From nine rows on a step's o, gate/up and down projections are panel GEMMs
+    with the norm behind them: the first, middle and last sequence against the
+    oracle, as the smaller batches are checked."""
+    from tests.test_gpu_batch import _oracle_runs
+    from tests.test_gpu_engine import SMALL, _check_run, _prompt
+    from tilefoundry_amd.qwen3 import synthetic_weights
+    from tilefoundry_amd.qwen3.batch_engine import BatchEngine
+
+    w = synthetic_weights(SMALL, seed=2, norms="ones")
+    prompts = [_prompt(3 + b % 5, SMALL.vocab_size, seed=b) for b in range(batch)]
+    eng = BatchEngine(SMALL, w, batch=batch, device=gpu_device, max_new=12, prompt_room=8)
+    run = eng.generate(prompts, 12, record_logits=True)
+    some = [0, batch // 2, batch - 1]
+    for b, orc in zip(some, _oracle_runs(SMALL, w, [prompts[b] for b in some], 12)):
+        seq = type("Run", (), {"tokens": run.tokens[b], "logits": run.logits[b]})
+        _check_run(seq, orc, 12, strict=False)

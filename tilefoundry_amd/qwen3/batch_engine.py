@@ -7,8 +7,8 @@ The batch-1 engine's structure (``engine.py``; the reference's
   shared page pool per layer (``[B * pages][HKV][16][D]`` bf16, a seeded
   permutation so every sequence's pages are scattered through the pool);
 * the projections are skinny GEMMs on the matrix cores
-  (``tfd_gemm_skinny_bf16``: M = batch rows, 16x16x32 bf16 MFMA), the norms run
-  row by row, and attention runs per (split, kv head, sequence);
+  (``tfd_gemm_skinny_bf16``: M = batch rows, 16x16x32 bf16 MFMA; from nine rows on,
+  panel GEMMs whose sums the next norm adds), the norms run row by row, and attention runs per (split, kv head, sequence);
 * the whole step -- every layer, the head, the per-sequence pick and the next
   embeddings -- is recorded once into a HIP graph and replayed; the last kernel
   feeds each sequence its next prompt token while its prompt lasts and its pick
@@ -177,6 +177,13 @@ class BatchEngine:
         # skinny-GEMM work: tile counters (kept at zero by the library) and the
         # f32 partial tiles of GEMMs that split K; 8 MiB covers every projection
         self.work = z(1 << 21, dtype=f32)
+        # From nine rows on, the output and down projections leave K-split sums that the
+        # next norm adds (two launches for three, and no hand-off inside the GEMM).  A
+        # step of eight layers of Qwen3-1.7B: 578 against 648 us at 32 rows, 534 / 553
+        # at 16, 518 / 520 at 8; at one row 503 / 464, where the skinny GEMM wastes less.
+        self.panels = B > 8
+        self.part = z(max(self._lib.tfd_panel_gemm_slices(B, K, self.H) for K in
+                          (self.QD, self.I)) * B * self.H, dtype=f32)
 
     def _stream(self) -> int:
         return torch.cuda.current_stream(self.device).cuda_stream
@@ -189,13 +196,25 @@ class BatchEngine:
                                        0 if resid is None else resid.shape[-1], ptr(out), ldo,
                                        ptr(self.work), self.work.numel(), s)
 
+    def _norm(self, x, gamma, s):
+        """xn = the rows' RMSNorm, in operand order."""
+        self._lib.tfd_rmsnorm_rows_bf16(ptr(x), self.H, ptr(gamma), ptr(self.xn), 0, self.B,
+                                        self.H, self.eps, 1, s)
+
+    def _project(self, x, w, K, resid, out, gamma, s):
+        """out = resid + x @ w^T, and its norm by *gamma* in xn (model.py:213-225)."""
+        L, B, H = self._lib, self.B, self.H
+        L.tfd_panel_gemm_bf16(ptr(x), ptr(w), B, K, H, _lib.PANEL_PARTIAL, ptr(self.part), s)
+        L.tfd_panel_add_norm(ptr(self.part), L.tfd_panel_gemm_slices(B, K, H), ptr(resid),
+                             ptr(out), ptr(gamma), ptr(self.xn), B, H, self.eps, s)
+
     def _layer(self, i: int, s: int):
-        """One decoder layer (model.py:236-266) for every sequence."""
+        """One decoder layer (model.py:236-266) for every sequence; xn holds its
+        normalised input and takes the next layer's (or the head's)."""
         L, w = self._lib, self.layers[i]
         B, H, I, D = self.B, self.H, self.I, self.D
         x_in, x_out = self.hid_rows[i], self.hid_rows[i + 1]
-        L.tfd_rmsnorm_rows_bf16(ptr(x_in), H, ptr(w["gamma_in"]), ptr(self.xn), 0, B, H,
-                                self.eps, 1, s)
+        gamma = self.layers[i + 1]["gamma_in"] if i + 1 < self.L else self.gamma_final
         self._gemm(self.xn, w["w_qkv"], H, self.qkv_n, _lib.EPI_STORE, None, self.qkv,
                    self.qkv_n, s)
         L.tfd_attn_rope_scores_paged_batched(
@@ -210,20 +229,27 @@ class BatchEngine:
             self.score_stride, ptr(self.smax), ptr(self.snew), ptr(self.psum), ptr(self.pout),
             self.nsplit, self.split_tiles, ptr(self.counters), ptr(self.attn),
             ptr(self.err), s)
-        self._gemm(self.attn, w["w_o"], self.QD, H, _lib.EPI_RESID, x_in, self.h1, H,
-                   s)
-        L.tfd_rmsnorm_rows_bf16(ptr(self.h1), H, ptr(w["gamma_post"]), ptr(self.xn), 0, B, H,
-                                self.eps, 1, s)
-        self._gemm(self.xn, w["w_gu"], H, 2 * I, _lib.EPI_SWIGLU, None, self.hmid, 0, s)
-        self._gemm(self.hmid, w["w_down"], I, H, _lib.EPI_RESID, self.h1, x_out, H, s)
+        if not self.panels:
+            self._gemm(self.attn, w["w_o"], self.QD, H, _lib.EPI_RESID, x_in, self.h1, H, s)
+            self._norm(self.h1, w["gamma_post"], s)
+            self._gemm(self.xn, w["w_gu"], H, 2 * I, _lib.EPI_SWIGLU, None, self.hmid, 0, s)
+            self._gemm(self.hmid, w["w_down"], I, H, _lib.EPI_RESID, self.h1, x_out, H, s)
+            self._norm(x_out, gamma, s)
+            return
+        self._project(self.attn, w["w_o"], self.QD, x_in, self.h1, w["gamma_post"], s)
+        if L.tfd_panel_gemm_slices(B, H, 2 * I) == 1:
+            L.tfd_panel_gemm_bf16(ptr(self.xn), ptr(w["w_gu"]), B, H, 2 * I, _lib.PANEL_SWIGLU,
+                                  ptr(self.hmid), s)
+        else:
+            self._gemm(self.xn, w["w_gu"], H, 2 * I, _lib.EPI_SWIGLU, None, self.hmid, 0, s)
+        self._project(self.hmid, w["w_down"], I, self.h1, x_out, gamma, s)
 
     def _step(self):
         s = self._stream()
+        L, B, H = self._lib, self.B, self.H
+        self._norm(self.hid, self.layers[0]["gamma_in"], s)
         for i in range(self.L):
             self._layer(i, s)
-        L, B, H = self._lib, self.B, self.H
-        L.tfd_rmsnorm_rows_bf16(ptr(self.hid_rows[self.L]), H, ptr(self.gamma_final),
-                                ptr(self.xn), 0, B, H, self.eps, 1, s)
         self._gemm(self.xn, self.w_head, H, self.V, _lib.EPI_LOGITS, None, self.logits,
                    self.V, s)
         self.picker(self.logits, self.V, self.pick, self.pos, s)
