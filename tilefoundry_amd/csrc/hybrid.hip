@@ -12,8 +12,9 @@
 // Batch rows are sequences (one token each); the projections around these
 // kernels are the skinny GEMMs (tfd_gemm_skinny_bf16 / _fp8).
 
-#include "hybrid_common.h"
 #include "host_common.h"
+#include "hybrid_common.h"
+#include "panel.h"
 #include "tf_decode.h"
 #include "tf_hybrid.h"
 
@@ -313,6 +314,171 @@ __global__ __launch_bounds__(kBlock) void k_moe_down(MoeArgs a) {
       u32x4 hr[kC];
       hload(t, hr);
       products(t, hr);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same two projections on the matrix cores, over row-major e4m3fn weights
+// (bf16 policy), for more rows than lane-wise sums per (entry, weight row) keep
+// up with: those decode every weight again for each entry.  A wave takes 16 gate
+// and 16 up rows (or 32 rows of the down projection), 128 values of each at a
+// time, requested a piece ahead and turned into operands through LDS of its own;
+// up to 32 entries of the group are the columns and pass through LDS the block
+// shares, so a weight is read and decoded once for all of them.
+// Bound: LDS and the waits between a piece's load and its use (about 60% of what
+// the weights' stream could do).  Granite's experts (72 of 768 x 4096), experts of
+// 32 rows 297 -> 184 us, 24 rows 248 -> 168, 17 rows 204 -> 178; 256-value pieces
+// 190, 185, 191 (fewer blocks per compute unit).  The bf16 experts' sums are as
+// fast by lanes (Qwen3.5's: 16 rows 123 against 130 us, 32 rows 196 / 192).
+// ---------------------------------------------------------------------------
+constexpr int kMtRows = 32;                  // entries per pass
+constexpr int kMtK = 128;                    // K values per piece
+constexpr int kMtLd = kMtK + 16;             // LDS bytes between weight rows
+constexpr int kMtXs = kMtK + 8;              // LDS values between entries
+struct MoeRowTile {
+  u32x4 raw[2];
+  __device__ __forceinline__ void load(const void* w, int64_t row0, int K, int c, int lane) {
+    const uint8_t* p = (const uint8_t*)w + (row0 + lane / 8) * K + c * kMtK + (lane % 8) * 16;
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      raw[v] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + (int64_t)8 * v * K));
+  }
+  __device__ __forceinline__ void stage(uint8_t* s, int lane) const {
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      *reinterpret_cast<u32x4*>(s + (8 * v + lane / 8) * kMtLd + (lane % 8) * 16) = raw[v];
+  }
+  // lane l: row l % 16, K values 32 v + 8 (l / 16) .. +7
+  static __device__ __forceinline__ u32x4 operand(const uint8_t* s, int v, int lane) {
+    return fp8x8_to_bf16(*reinterpret_cast<const u32x2*>(s + (lane % 16) * kMtLd + 32 * v +
+                                                         8 * (lane / 16)));
+  }
+};
+
+template <bool kDown>
+__global__ __launch_bounds__(kBlock) void k_moe8_rows(MoeArgs a) {
+  __shared__ __align__(16) bf16 xs[kMtRows * kMtXs];
+  __shared__ __align__(16) uint8_t ws[kWavesPerBlock * 2 * 16 * kMtLd];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  Group g;
+  if (!moe_group<0>(a, g)) return;
+  const int width = g.shared ? a.IS : a.I;
+  const int N = kDown ? a.H : width, K = kDown ? width : a.H;
+  constexpr int kCols = kDown ? 32 : 16;                   // output columns per wave
+  if ((int)blockIdx.x * kWavesPerBlock * kCols >= N) return;
+  const int c0 = (blockIdx.x * kWavesPerBlock + wave) * kCols;
+  const bool on = c0 < N;
+  const int cA = on ? c0 : 0;
+  const void *w0, *w1;
+  int64_t rA, rB;                                          // first weight row of each half
+  const float *sA, *sB;
+  if (kDown) {
+    w0 = w1 = g.shared ? a.w_sout : a.w_down;
+    rA = (g.shared ? 0 : (int64_t)g.e * a.H) + cA;
+    rB = rA + 16;
+    sA = (g.shared ? a.s_sout : a.s_down) + rA;
+    sB = sA + 16;
+  } else {
+    w0 = g.shared ? a.w_sin : a.w_gate;
+    w1 = g.shared ? a.w_sin : a.w_up;
+    rA = (g.shared ? 0 : (int64_t)g.e * a.I) + cA;
+    rB = g.shared ? a.IS + cA : rA;
+    sA = (g.shared ? a.s_sin : a.s_gate) + rA;
+    sB = (g.shared ? a.s_sin : a.s_up) + rB;
+  }
+  uint8_t* wsA = ws + wave * 2 * 16 * kMtLd;               // this wave's alone
+  uint8_t* wsB = wsA + 16 * kMtLd;
+  const int chunks = K / kMtK;
+  const int r = lane % 16, kq = lane / 16;
+  for (int t0 = 0; t0 < g.count; t0 += kMtRows) {
+    const int rows = min(kMtRows, g.count - t0), sub = (rows + 15) / 16;
+    MoeRowTile tA, tB;
+    auto load_w = [&](int c) {
+      tA.load(w0, rA, K, c, lane);
+      tB.load(w1, rB, K, c, lane);
+    };
+    load_w(0);                                             // before the entries are known
+    __builtin_amdgcn_sched_barrier(0);
+    // this thread's 16 bytes of two entries; rows past the count are left as they
+    // are in LDS (a column of the product is one entry's, and theirs are not stored)
+    const bf16* xp[2];
+    bool xon[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int t = i * 16 + tid / 16;
+      int b, slot;
+      xon[i] = t < rows;
+      moe_entry(a, g, t0 + min(t, rows - 1), b, slot);
+      xp[i] = (kDown ? a.hidden + ((int64_t)b * (a.k + 1) + slot) * a.IM
+                     : a.x + (int64_t)b * a.H) + (tid % 16) * 8;
+    }
+    u32x4 xr[2];
+    auto load_x = [&](int c) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (xon[i]) xr[i] = load16(xp[i] + c * kMtK);
+    };
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    load_x(0);
+    for (int c = 0; c < chunks; ++c) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (xon[i])
+          *reinterpret_cast<u32x4*>(&xs[(i * 16 + tid / 16) * kMtXs + (tid % 16) * 8]) = xr[i];
+      tA.stage(wsA, lane);
+      tB.stage(wsB, lane);
+      if (c + 1 < chunks) {
+        load_x(c + 1);
+        load_w(c + 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int v = 0; v < kMtK / 32; ++v) {
+        const u32x4 opA = MoeRowTile::operand(wsA, v, lane);
+        const u32x4 opB = MoeRowTile::operand(wsB, v, lane);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (i < sub) {
+            const u32x4 x =
+                *reinterpret_cast<const u32x4*>(&xs[(i * 16 + r) * kMtXs + 32 * v + 8 * kq]);
+            acc[i][0] = mfma(opA, x, acc[i][0]);
+            acc[i][1] = mfma(opB, x, acc[i][1]);
+          }
+      }
+      __syncthreads();
+    }
+    if (!on) continue;
+    float scA[4], scB[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      scA[q] = sA[4 * kq + q];
+      scB[q] = sB[4 * kq + q];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (i * 16 + r >= rows) continue;
+      int b, slot;
+      moe_entry(a, g, t0 + i * 16 + r, b, slot);
+      const int64_t at = (int64_t)b * (a.k + 1) + slot;
+      if (kDown) {
+        float* o = a.partial + at * a.H + cA + 4 * kq;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          o[q] = rbf(acc[i][0][q] * scA[q]);
+          o[16 + q] = rbf(acc[i][1][q] * scB[q]);
+        }
+      } else {
+        float h[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          h[q] = rbf(silu_f(rbf(acc[i][0][q] * scA[q]))) * rbf(acc[i][1][q] * scB[q]);
+        *reinterpret_cast<u32x2*>(a.hidden + at * a.IM + cA + 4 * kq) =
+            u32x2{pack2(h[0], h[1]), pack2(h[2], h[3])};
+      }
     }
   }
 }
@@ -1282,12 +1448,30 @@ int launch_moe8(const MoeArgs& a, hipStream_t s) {
   return launched("moe_experts_packed");
 }
 
+// k_moe8_rows takes whole pieces of K with 16-byte weight loads, and from 17 rows
+// on (up to 16 the engine's experts are packed, which is faster still)
+bool moe8_rows_fits(const MoeArgs& a) {
+  const uintptr_t p = (uintptr_t)a.w_gate | (uintptr_t)a.w_up | (uintptr_t)a.w_down |
+                      (uintptr_t)a.w_sin | (uintptr_t)a.w_sout;
+  return a.B > kM8 && a.H % kMtK == 0 && a.I % kMtK == 0 && a.IS % kMtK == 0 && (p & 15) == 0;
+}
+
 template <bool kFp8, bool kF32>
 int launch_moe(const MoeArgs& a, hipStream_t s) {
   // picked experts at most min(E, B k), plus the shared one
   const int np = a.E < a.B * a.k ? a.E : a.B * a.k;
   const dim3 g3((a.H + kBlock - 1) / kBlock, a.B);
   launch_group(a, s);
+  if (kFp8 && moe8_rows_fits(a)) {
+    const int width = a.I > a.IS ? a.I : a.IS;
+    constexpr int kGu = 16 * kWavesPerBlock, kDn = 32 * kWavesPerBlock;   // columns per block
+    hipLaunchKernelGGL((k_moe8_rows<false>), dim3((width + kGu - 1) / kGu, np + 1),
+                       dim3(kBlock), 0, s, a);
+    hipLaunchKernelGGL((k_moe8_rows<true>), dim3((a.H + kDn - 1) / kDn, np + 1), dim3(kBlock),
+                       0, s, a);
+    hipLaunchKernelGGL((k_moe_mix<kF32>), g3, dim3(kBlock), 0, s, a);
+    return launched("moe_experts");
+  }
   // gate/up in one launch; the down projections in one launch when the shared
   // expert is as wide as the routed ones, else one for each width (a lane's
   // chunk registers are sized by the width)
