@@ -363,21 +363,26 @@ __global__ __launch_bounds__(kBlock) void k_panel_gqa_append(
 // Causal attention of a prompt pass (model.py:190-212) over the paged cache,
 // which already holds the pass's own keys and values.
 //
-// A block takes one tile of consecutive rows of a sequence (128 / G of them) and
-// one kv head: 128 (query head, row) columns, 32 per wave, past the context in
+// A block takes one tile of consecutive rows of a sequence (64 CT / G of them) and
+// one kv head: 64 CT (query head, row) columns, 16 CT per wave, past the context in
 // tiles of 64 positions.  S^T = K Q^T puts four consecutive positions of one
 // column in a lane; packed, that is the B operand of O^T = V^T P^T as it stands
 // if V^T's positions are stored in the same order, so the probabilities never
 // leave their lane.  K and V tiles are read once per block, prefetched into
 // registers while the tile before is used, V transposed on its way into LDS.
 //
-// Bound: the softmax's VALU work (about 1,500 cycles a tile and wave against 1,024 of
-// matrix products and as many of LDS).  4,001 rows take 214 us a layer (302 with a
-// page-table read in front of each load, expf, and an unconditional rescale).
+// Bound: one wave's chain through a tile (LDS reads, products, softmax, products) with
+// three waves per SIMD to cover it; of the busy cycles 45% are VALU, 18% matrix cores
+// and a third LDS.  4,000 rows take 141 us a layer, eight prompts of 88-700 tokens 27,
+// 91 rows 8.7.  What mattered: LDS in operand order (row-major tiles spent three
+// quarters of their LDS cycles in bank conflicts: 213, 35 and 10.6 us); 16 columns a
+// wave, whose registers let three blocks share a compute unit and whose tiles are half as
+// long (32 columns and two blocks: 164, 33 and 11.9); page ids read a tile ahead, and a
+// rescale only when a maximum moves (302 us before both, with 32 columns).
 //
 // The decode kernels it takes the place of re-read every cached key for each row: a
-// 4,001-token prompt through eight layers took 123.0 ms, here 6.02 ms; 91 tokens
-// 2.16 and 1.01 ms, eight prompts of 88-700 tokens 51.4-71 and 5.29 ms (each with
+// 4,001-token prompt through eight layers took 123.0 ms, here 4.88 ms; 91 tokens
+// 2.18 and 0.99 ms, eight prompts of 88-700 tokens 51.4-71 and 4.07 ms (each with
 // one decode step).
 //
 // Rounding: s = bf16(q . k), p = bf16(exp(bf16(s - m))) against the running
@@ -417,7 +422,7 @@ __device__ __forceinline__ void split3(const f32x4& a, const f32x4& b, u32x4 (&o
 enum PanelAttnPolicy { kAttnDense = 0, kAttnGranite = 1, kAttnF32 = 2 };
 
 template <int D, int G, int CT, int kPol>
-__global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
+__global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_panel_attn(
     const void* __restrict__ q_in, const PanelTile* __restrict__ tiles, int heads, int kv_heads,
     const int* __restrict__ page_table, int max_pages, const bf16* __restrict__ kpool,
     const bf16* __restrict__ vpool, int num_pages, float scale,
@@ -426,13 +431,15 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
   constexpr int QT = 64 * CT / G;            // rows of a tile
   constexpr int kQ = kPol == kAttnF32 ? 3 : 1;   // operands per query / probability
   constexpr int DS = D / 32, DT = D / 16;    // k steps of q.k, 16-row tiles of V^T
-  constexpr int KS = D + 8, VS = 64 + 8;     // LDS row strides (bf16)
   constexpr int kCh = D / 8;                 // 16-byte chunks of a head row
   constexpr int kKPass = 64 * kCh / kBlock;  // K loads per thread and tile
   constexpr int kVThr = 16 * kCh;            // pieces of V: 4 positions x 8 dims each
   constexpr int kVPass = kVThr > kBlock ? kVThr / kBlock : 1;
-  __shared__ __align__(16) bf16 ks[64 * KS];
-  __shared__ __align__(16) bf16 vt[D * VS];
+  // Both tiles lie in operand order, 1 KiB per 16 x 32 block.  Lane l's 16 bytes are at
+  // l ^ l / 16 ^ 4 (step % 4) in K and at l ^ (block % 8) in V^T, so that the lanes of a
+  // write (pieces of a few rows) fall on as many banks as those of a read.
+  __shared__ __align__(16) uint8_t ks[64 * D * 2];
+  __shared__ __align__(16) uint8_t vt[64 * D * 2];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int r = lane & 15, kq = lane >> 4;
@@ -479,6 +486,7 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
   const int vc = tid % kCh;                  // V: 8-dim chunk; position group tid / kCh + ..
   // lane l holds the id of a tile's page l % 4, read a tile ahead of the loads that
   // need it (a page-table read in front of every load made a tile five round trips)
+  auto v_at = [](int i) { return 32 * (i >> 3) + 16 * (i & 1) + 4 * ((i >> 1) & 3); };
   auto load_tile = [&](int j0, int pid) {
 #pragma unroll
     for (int i = 0; i < kKPass; ++i) {
@@ -490,7 +498,7 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
     if (kVThr >= kBlock || tid < kVThr) {
 #pragma unroll
       for (int g = 0; g < kVPass; ++g) {
-        const int at = 4 * ((tid + g * kBlock) / kCh), p = j0 + at;
+        const int at = v_at((tid + g * kBlock) / kCh), p = j0 + at;
         const int page = __shfl(pid, at / kPage, kWave);
         const bf16* v0 = vpool + (((int64_t)page * kv_heads + h) * kPage + p % kPage) * D + vc * 8;
         // positions past the last row hold anything (their p is 0): their V reads as 0
@@ -506,7 +514,8 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
 #pragma unroll
     for (int i = 0; i < kKPass; ++i) {
       const int c = tid + i * kBlock;
-      *reinterpret_cast<u32x4*>(&ks[(c / kCh) * KS + (c % kCh) * 8]) = kr[i];
+      const int p = c / kCh, s = c % kCh / 4, l = 16 * (c % 4) + p % 16;
+      *reinterpret_cast<u32x4*>(&ks[(p / 16 * DS + s) * 1024 + (l ^ (c % kCh & 15)) * 16]) = kr[i];
     }
     if (kVThr >= kBlock || tid < kVThr) {
       // positions in the order the probabilities come in: within 32, position
@@ -514,7 +523,7 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
 #pragma unroll
       for (int g = 0; g < kVPass; ++g) {
         const int vg = (tid + g * kBlock) / kCh;
-        const int at = 32 * (vg >> 3) + 8 * (vg & 3) + 4 * ((vg >> 2) & 1);
+        const int at = (vc / 2 * 2 + (vg >> 3)) * 1024 + 8 * (vg & 1);
         auto word = [&](int i, int d) {
           const u32x4 v = vr[g][i];
           return (d >> 1) == 0 ? v.x : (d >> 1) == 1 ? v.y : (d >> 1) == 2 ? v.z : v.w;
@@ -522,7 +531,8 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
           const uint32_t sel = (d & 1) ? 0x07060302u : 0x05040100u;
-          *reinterpret_cast<u32x2*>(&vt[(vc * 8 + d) * VS + at]) =
+          const int l = 16 * ((vg >> 1) & 3) + 8 * (vc % 2) + d;
+          *reinterpret_cast<u32x2*>(&vt[at + (l ^ (vc / 2 & 7)) * 16]) =
               u32x2{__builtin_amdgcn_perm(word(1, d), word(0, d), sel),
                     __builtin_amdgcn_perm(word(3, d), word(2, d), sel)};
         }
@@ -562,7 +572,8 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
     for (int s = 0; s < DS; ++s)
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-        const u32x4 kf = *reinterpret_cast<const u32x4*>(&ks[(16 * p + r) * KS + 32 * s + 8 * kq]);
+        const u32x4 kf =
+            *reinterpret_cast<const u32x4*>(&ks[(p * DS + s) * 1024 + (lane ^ kq ^ 4 * (s & 3)) * 16]);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -644,7 +655,8 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? 2 : 1) void k_panel_attn(
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const u32x4 vf = *reinterpret_cast<const u32x4*>(&vt[(16 * dt + r) * VS + 32 * kk + 8 * kq]);
+        const u32x4 vf =
+            *reinterpret_cast<const u32x4*>(&vt[(dt * 2 + kk) * 1024 + (lane ^ (dt & 7)) * 16]);
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
@@ -930,7 +942,7 @@ int tfd_panel_qkv_append(const float* part, int slices, int M, int heads, int kv
   return launched("panel_qkv_append");
 }
 
-int tfd_panel_attn_rows(int group) { return group > 0 && group <= 8 ? 128 / group : 0; }
+int tfd_panel_attn_rows(int group) { return group > 0 && group <= 8 ? 64 / group : 0; }
 
 int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, int kv_heads,
                    int head_dim, const int32_t* page_table, int max_pages, const void* k_pool,
@@ -944,7 +956,7 @@ int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, i
   const dim3 grid(kv_heads, ntiles);
   auto s = (hipStream_t)stream;
 #define TFD_PANEL_ATTN(D, GG)                                                                   \
-  hipLaunchKernelGGL((k_panel_attn<D, GG, 2, kAttnDense>), grid, dim3(kBlock), 0, s, q,         \
+  hipLaunchKernelGGL((k_panel_attn<D, GG, 1, kAttnDense>), grid, dim3(kBlock), 0, s, q,         \
                      (const PanelTile*)tiles, heads, kv_heads, page_table, max_pages,           \
                      (const bf16*)k_pool, (const bf16*)v_pool, num_pages, 1.f, nullptr, nullptr, \
                      (bf16*)out, err)
