@@ -14,7 +14,7 @@
 // Rounding is the decode kernels' (hybrid.hip), per policy.
 //
 // Measured (four layers, prompt to first logits, one sequence): Qwen3.5 at 250 tokens
-// 58.4 ms walked, 1.93 ms in a pass; Granite at 190 tokens 65.5 and 1.89 ms.
+// 58.4 ms walked, 1.92 ms in a pass; Granite at 190 tokens 65.9 and 1.78 ms.
 
 #include "host_common.h"
 #include "hybrid_common.h"
@@ -69,11 +69,12 @@ __global__ __launch_bounds__(kBlock) void k_panel_halves(const float* __restrict
 
 // ---------------------------------------------------------------------------
 // Residual stream and next norm, a block per row.  The experts' mix adds the slots
-// in slot order, then the shared expert, as k_moe_mix does.
+// in slot order, then the shared expert, as k_moe_mix does; five slots' loads are in
+// flight together (190 rows of ten slots, 4,096 columns: 20.2 us one by one, 15.8).
 // ---------------------------------------------------------------------------
 template <bool kF32, bool kMoe>
 __global__ __launch_bounds__(kBlock) void k_panel_mix(TfdPanelMixArgs a) {
-  constexpr int kMax4 = 8;                   // n <= 8192
+  constexpr int kMax4 = 8, kSlots = 5;       // n <= 8192; slots of the mix per round trip
   __shared__ float red[kWavesPerBlock];
   const int64_t m = blockIdx.x;
   const int tid = threadIdx.x, n = a.n, n4 = n / 4;
@@ -115,13 +116,22 @@ __global__ __launch_bounds__(kBlock) void k_panel_mix(TfdPanelMixArgs a) {
         for (int e = 0; e < 4; ++e) y[e] = rbf(y[e]);
         if (kMoe) {
           f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-          for (int s = 0; s < a.k; ++s) {
-            const u32x2 w = *reinterpret_cast<const u32x2*>((const bf16*)a.d +
-                                                            (m * a.k + s) * n + c);
-            const float wt = a.weights[m * a.k + s];
-            const float d[4] = {bf_lo(w.x), bf_hi(w.x), bf_lo(w.y), bf_hi(w.y)};
+          for (int s0 = 0; s0 < a.k; s0 += kSlots) {       // their loads in flight together
+            u32x2 w[kSlots];
+            float wt[kSlots];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] += kF32 ? d[e] * wt : rbf(d[e] * wt);
+            for (int s = 0; s < kSlots; ++s) {
+              const int64_t at = m * a.k + min(s0 + s, a.k - 1);
+              w[s] = *reinterpret_cast<const u32x2*>((const bf16*)a.d + at * n + c);
+              wt[s] = a.weights[at];
+            }
+#pragma unroll
+            for (int s = 0; s < kSlots; ++s)
+              if (s0 + s < a.k) {
+                const float d[4] = {bf_lo(w[s].x), bf_hi(w[s].x), bf_lo(w[s].y), bf_hi(w[s].y)};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += kF32 ? d[e] * wt[s] : rbf(d[e] * wt[s]);
+              }
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -558,14 +568,19 @@ __global__ __launch_bounds__(kBlock) void k_pmamba_conv(TfdPanelMambaArgs a) {
 
 // The state update over the sequence's T tokens: a block takes 32 of a head's 64 state
 // rows, eight lanes to a row, sixteen columns each in registers (columns 32 j + 4 ng
-// + e); B and C come through LDS, sixteen tokens at a time.
+// + e); bf16(dt B) and C come through LDS, sixteen tokens at a time and read a token
+// ahead.
+// Bound: the VALU, one wave to a SIMD (eleven operations a state and token with dt B
+// formed by every row and one value to a conversion: 92 us for 190 tokens; six with two
+// values to a conversion and C's products summed in pairs: 71, 0.37 a token).
 __global__ __launch_bounds__(kBlock) void k_pmamba_scan(TfdPanelMambaArgs a) {
   const int h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
   const int pl = tid / 8, ng = tid % 8, p = blockIdx.x * 32 + pl;
   const int exp_ = a.heads * kMP;
   const int64_t m0 = (int64_t)b * a.T;
-  __shared__ __align__(16) float b_s[kScanT][kMN], c_s[kScanT][kMN];
-  __shared__ float x_s[kScanT][32], g_s[kScanT][2];
+  __shared__ __align__(16) float b_s[kScanT][kMN];       // bf16(dt B)
+  __shared__ __align__(16) bf16 c_s[kScanT][kMN];
+  __shared__ float x_s[kScanT][32], g_s[kScanT];
   float* st = a.state + (((int64_t)b * a.heads + h) * kMP + p) * kMN + 4 * ng;
   float s[16];
 #pragma unroll
@@ -577,49 +592,76 @@ __global__ __launch_bounds__(kBlock) void k_pmamba_scan(TfdPanelMambaArgs a) {
   const float dsk = bf2f(((const bf16*)a.d_skip)[h]);
   u32x4 bcr[2];
   bf16 xr[2];
-  float gr = 0.f;
+  float dtr[2], gr = 0.f;
   auto load = [&](int t0) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int c = tid + i * kBlock;        // B | C: 32 pieces of 8 a token
       const int64_t m = m0 + min(t0 + c / 32, a.T - 1);
+      dtr[i] = a.gates[(m * a.heads + h) * 2 + 1];
       bcr[i] = load16((const bf16*)a.bc + m * 2 * kMN + (c % 32) * 8);
       xr[i] = ((const bf16*)a.x)[m * exp_ + h * kMP + blockIdx.x * 32 + c % 32];
     }
-    if (tid < 2 * kScanT)
-      gr = a.gates[((m0 + min(t0 + tid / 2, a.T - 1)) * a.heads + h) * 2 + tid % 2];
+    if (tid < kScanT) gr = a.gates[((m0 + min(t0 + tid, a.T - 1)) * a.heads + h) * 2];
   };
   load(0);
   for (int t0 = 0; t0 < a.T; t0 += kScanT) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int c = tid + i * kBlock, part = c % 32;
-      float* dst = part < 16 ? &b_s[c / 32][part * 8] : &c_s[c / 32][(part - 16) * 8];
-      *reinterpret_cast<f32x4*>(dst) = f32x4{bf_lo(bcr[i].x), bf_hi(bcr[i].x), bf_lo(bcr[i].y),
-                                             bf_hi(bcr[i].y)};
-      *reinterpret_cast<f32x4*>(dst + 4) = f32x4{bf_lo(bcr[i].z), bf_hi(bcr[i].z),
-                                                 bf_lo(bcr[i].w), bf_hi(bcr[i].w)};
+      if (part < 16) {
+        const float dt = dtr[i];
+        float* dst = &b_s[c / 32][part * 8];
+        *reinterpret_cast<f32x4*>(dst) =
+            f32x4{rbf(dt * bf_lo(bcr[i].x)), rbf(dt * bf_hi(bcr[i].x)),
+                  rbf(dt * bf_lo(bcr[i].y)), rbf(dt * bf_hi(bcr[i].y))};
+        *reinterpret_cast<f32x4*>(dst + 4) =
+            f32x4{rbf(dt * bf_lo(bcr[i].z)), rbf(dt * bf_hi(bcr[i].z)),
+                  rbf(dt * bf_lo(bcr[i].w)), rbf(dt * bf_hi(bcr[i].w))};
+      } else {
+        *reinterpret_cast<u32x4*>(&c_s[c / 32][(part - 16) * 8]) = bcr[i];
+      }
       x_s[c / 32][c % 32] = bf2f(xr[i]);
     }
-    if (tid < 2 * kScanT) g_s[tid / 2][tid % 2] = gr;
+    if (tid < kScanT) g_s[tid] = gr;
     __syncthreads();
     if (t0 + kScanT < a.T) load(t0 + kScanT);
     const int n = min(kScanT, a.T - t0);
-    for (int t = 0; t < n; ++t) {
-      const float decay = g_s[t][0], dt = g_s[t][1], xp = x_s[t][pl];
-      float rd = 0.f;
+    f32x4 bn[4];                             // a token ahead of its use
+    u32x2 cn[4];
+    float dn, xn;
+    auto fetch = [&](int t) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const f32x4 b4 = *reinterpret_cast<const f32x4*>(&b_s[t][32 * j + 4 * ng]);
-        const f32x4 c4 = *reinterpret_cast<const f32x4*>(&c_s[t][32 * j + 4 * ng]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float& u = s[4 * j + e];
-          u = u * decay + rbf(rbf(dt * b4[e]) * xp);
-          rd = fmaf(rbf(u), c4[e], rd);
-        }
+        bn[j] = *reinterpret_cast<const f32x4*>(&b_s[t][32 * j + 4 * ng]);
+        cn[j] = *reinterpret_cast<const u32x2*>(&c_s[t][32 * j + 4 * ng]);
       }
-      rd = group_sum<8>(rd);
+      dn = g_s[t];
+      xn = x_s[t][pl];
+    };
+    fetch(0);
+    for (int t = 0; t < n; ++t) {
+      const float decay = dn, xp = xn;
+      f32x4 bt[4];
+      u32x2 ct[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        bt[j] = bn[j];
+        ct[j] = cn[j];
+      }
+      fetch(min(t + 1, kScanT - 1));
+      float r2[2] = {0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {        // two states per conversion and per dot
+          float &u = s[4 * j + 2 * i], &w = s[4 * j + 2 * i + 1];
+          const uint32_t in = pack2(bt[j][2 * i] * xp, bt[j][2 * i + 1] * xp);
+          u = u * decay + bf_lo(in);
+          w = w * decay + bf_hi(in);
+          r2[i] = dot2(pack2(u, w), i == 0 ? ct[j].x : ct[j].y, r2[i]);
+        }
+      const float rd = group_sum<8>(r2[0] + r2[1]);
       if (ng == 0)
         ((bf16*)a.y)[(m0 + t0 + t) * exp_ + h * kMP + p] = f2bf(rbf(rd) + rbf(xp * dsk));
     }
