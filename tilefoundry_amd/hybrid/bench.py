@@ -501,7 +501,7 @@ def main(argv=None) -> int:
     ap.add_argument("--steps", type=int, default=256, help="c4-step / c5-step: timed steps")
     ap.add_argument("--context", choices=("drawn", "walk"), default="drawn",
                     help="c5-step: the contexts drawn into the caches and states (default) or "
-                         "built by prefill from random prompts (about 53 s at 8,192 tokens)")
+                         "built by prefill from random prompts")
     ap.add_argument("--ctx", type=int, default=8192, help="c5-step: context length")
     ap.add_argument("--path", choices=("auto", "small", "mfma"), default="auto",
                     help="c4-step: the small-batch kernels (rows <= 4, the default there) or "
