@@ -97,3 +97,23 @@ def test_odd_sizes_are_walked(gpu_device):
     prompts = [[1, 2 + b, 3] for b in range(17)]
     eng.prefill(prompts)
     assert eng.pos.tolist() == [2] * 17 and eng.ids.tolist() == [3] * 17
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["qwen3_5", "granite"])
+def test_an_engine_that_prefilled_is_freed_when_dropped(gpu_device, model):
+    """The engine and its pass hold no cycle: its device memory goes with the last
+    reference, not with a later garbage collection."""
+    import gc
+    import weakref
+
+    eng = _engine(model, 1, gpu_device, 12)
+    gc.collect()
+    gc.disable()
+    try:
+        eng.prefill([list(range(1, 9))])
+        gone = weakref.ref(eng)
+        del eng
+        assert gone() is None
+    finally:
+        gc.enable()

@@ -18,6 +18,7 @@ state (or its keys and values); nothing reads what would follow.
 from __future__ import annotations
 
 import ctypes
+import weakref
 
 import numpy as np
 import torch
@@ -43,12 +44,18 @@ class _Pass:
     fp8: bool
 
     def __init__(self, eng):
-        self.e, self.cfg, self._lib = eng, eng.cfg, lib()
+        # the engine holds this pass: a strong reference back would keep both, and
+        # their device memory, until a garbage collection
+        self._eng, self.cfg, self._lib = weakref.ref(eng), eng.cfg, lib()
         self.B, self.H, self.k = eng.B, eng.cfg.hidden, eng.cfg.top_k
         self.dev = eng.device
         self.layers = [self._weights(w) for w in eng.layers]
         torch.cuda.synchronize(self.dev)
         self.rows = 0
+
+    @property
+    def e(self):
+        return self._eng()
 
     def _stream(self) -> int:
         return torch.cuda.current_stream(self.dev).cuda_stream
