@@ -211,6 +211,7 @@ def test_token_array_takes_what_a_prompt_may_be():
         int32_ids([(1 << 32) + 5])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("batch", [8, 9, 17, 32])
 def test_batch_step_on_both_sides_of_nine_rows(gpu_device, batch):
     """From nine rows on a step's o, gate/up and down projections are panel GEMMs
