@@ -138,6 +138,7 @@ def test_panel_attn(gpu_device, D, G, segs):
         rows = table[b].long()[at // 16]
         k[rows, :, at % 16] = float("nan")
         v[rows, :, at % 16] = float("nan")
+        table[b, -(-(p0 + n) // 16):] = -1  # nor are the pages past it
     M = sum(n for _, n in segs)
     q = (torch.randn(M, heads, D, generator=g, device=gpu_device) * D ** -0.5).to(bf)
     qt = L.tfd_panel_attn_rows(G)

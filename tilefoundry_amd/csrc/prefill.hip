@@ -452,8 +452,10 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_pa
   }
   const int* pt = page_table + (int64_t)tl.seq * max_pages;
   bool page_bad = false;
-  auto page_at = [&](int i) {                // entries past the table re-read its last
-    const int pg = pt[min(i, max_pages - 1)];
+  // entries past the last row's page need not be set (a table may be filled as the
+  // sequence grows): the tiles' read-ahead re-reads that one in their place
+  auto page_at = [&](int i) {
+    const int pg = pt[min(i, last / kPage)];
     const bool ok = pg >= 0 && pg < num_pages;
     page_bad |= !ok;
     return ok ? pg : 0;

@@ -8,7 +8,8 @@ The batch-1 engine's structure (``engine.py``; the reference's
   permutation so every sequence's pages are scattered through the pool);
 * the projections are skinny GEMMs on the matrix cores
   (``tfd_gemm_skinny_bf16``: M = batch rows, 16x16x32 bf16 MFMA; from nine rows on,
-  panel GEMMs whose sums the next norm adds), the norms run row by row, and attention runs per (split, kv head, sequence);
+  panel GEMMs whose sums the next norm adds), the norms run row by row, and
+  attention runs per (split, kv head, sequence);
 * the whole step -- every layer, the head, the per-sequence pick and the next
   embeddings -- is recorded once into a HIP graph and replayed; the last kernel
   feeds each sequence its next prompt token while its prompt lasts and its pick
