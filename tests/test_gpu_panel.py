@@ -1,5 +1,7 @@
 """Prompt-pass kernels (csrc/prefill.hip) against plain f32 references, at the
 sizes where tiles and passes end, and the cut of prompts into passes (CPU)."""
+import ctypes
+
 import pytest
 import torch
 
@@ -165,6 +167,93 @@ def test_panel_attn(gpu_device, D, G, segs):
         want = torch.einsum("hmp,phd->mhd", a, vc)
         assert (got[row:row + n] - want).abs().max() <= 3e-2 * want.abs().max()
         row += n
+
+
+def _attend(device, kind, poison=None):
+    """100 positions of one sequence through a prompt pass's attention -> [100][heads][D];
+    *poison* sets values of ([100][KV heads][D] keys, values) before the pass reads them."""
+    L = _lib.lib()
+    s = torch.cuda.current_stream().cuda_stream
+    n, bf, f32 = 100, torch.bfloat16, torch.float32
+    D, G, HKV = {"granite": (128, 4, 2), "f32": (256, 8, 1)}.get(kind) or (*kind, 2)
+    heads, pages = HKV * G, 7
+    g = torch.Generator(device=device).manual_seed(D + G)
+    rn = lambda *shape: torch.randn(*shape, generator=g, device=device)
+    z = lambda *shape, dtype=bf: torch.zeros(*shape, device=device, dtype=dtype)
+    q, k, v = rn(n, heads, D) * D ** -0.5, rn(n, HKV, D).to(bf), rn(n, HKV, D).to(bf)
+    if poison is not None:
+        poison(k, v)
+    table = torch.tensor([5, 0, 3, 6, 1, 4, 2], dtype=torch.int32, device=device)
+    kp, vp = z(pages, HKV, 16, D), z(pages, HKV, 16, D)
+    at = torch.arange(n, device=device)
+    qt = {"granite": _lib.PANEL_GQA_ROWS_BF16, "f32": _lib.PANEL_GQA_ROWS_F32}.get(kind) or \
+        L.tfd_panel_attn_rows(G)
+    tiles = torch.tensor([(t, min(qt, n - t), 0, t) for t in range(0, n, qt)],
+                         dtype=torch.int32, device=device)
+    out, err = z(128 * heads * D), z(1, dtype=torch.int32)
+    if kind not in ("granite", "f32"):
+        kp[table[at // 16].long(), :, at % 16] = k
+        vp[table[at // 16].long(), :, at % 16] = v
+        q = q.to(bf)
+        L.tfd_panel_attn(q.data_ptr(), tiles.data_ptr(), len(tiles), heads, HKV, D,
+                         table.data_ptr(), pages, kp.data_ptr(), vp.data_ptr(), pages,
+                         out.data_ptr(), err.data_ptr(), s)
+    else:
+        if kind == "f32":                   # (query, output gate) pairs
+            q = torch.stack((q, rn(n, heads, D)), 2)
+        proj = torch.cat((q.reshape(n, -1).to(bf), k.reshape(n, -1), v.reshape(n, -1)), 1)
+        pos, seq = at.to(torch.int32), z(n, dtype=torch.int32)
+        gam, cos, sin = z(D) + 1, z(112, 64) + 1, z(112, 64)
+        qw, gate, self_s = z(n * heads * D, dtype=f32), z(n * heads * D), z(n * heads, dtype=f32)
+        a = _lib.TfdPanelGqaArgs()
+        a.proj, a.ldp, a.M, a.err = proj.data_ptr(), proj.shape[1], n, err.data_ptr()
+        a.gamma_q, a.gamma_k = gam.data_ptr(), gam.data_ptr()
+        a.cos_table, a.sin_table, a.rope_rows, a.rot_dim = cos.data_ptr(), sin.data_ptr(), 112, 64
+        a.pos, a.seq, a.tiles, a.ntiles = pos.data_ptr(), seq.data_ptr(), tiles.data_ptr(), \
+            len(tiles)
+        a.page_table, a.max_pages, a.num_pages = table.data_ptr(), pages, pages
+        a.k_pool, a.v_pool, a.q, a.gate = kp.data_ptr(), vp.data_ptr(), qw.data_ptr(), \
+            gate.data_ptr()
+        a.self_scores, a.out, a.heads, a.kv_heads, a.head_dim = self_s.data_ptr(), \
+            out.data_ptr(), heads, HKV, D
+        a.scale, a.eps = (D ** -0.5, 1e-6) if kind == "f32" else (1.0, 1e-6)
+        a.policy = _lib.POLICY_F32 if kind == "f32" else _lib.POLICY_BF16
+        L.tfd_panel_gqa(ctypes.addressof(a), s)
+    torch.cuda.synchronize()
+    assert int(err.item()) == 0
+    return unpanel(out, n, heads * D).float().view(n, heads, D)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [(128, 2), (64, 2), (128, 1), "granite", "f32"], ids=str)
+@pytest.mark.parametrize("at", [0, 40, 70, 99])
+def test_panel_attn_rows_do_not_see_what_follows_them(gpu_device, kind, at):
+    """An infinite value, or a NaN key, at position *at*: the rows before it are what
+    they are without it, the rows from it on take it as a step takes it (an infinity of
+    that dimension alone; NaN throughout).  Rows taken position by position differ from
+    the tiles' by f32 orders, whose roundings test_panel_attn bounds: 3e-2 of the
+    largest value."""
+    clean = _attend(gpu_device, kind)
+    bar = 3e-2 * clean.abs().max()
+    rows = torch.arange(100, device=gpu_device)
+
+    def infinite(k, v):
+        v[at, 0, 5] = float("inf")
+
+    def nan_key(k, v):
+        k[at, 0] = float("nan")
+
+    mine = slice(0, clean.shape[1] // (1 if kind == "f32" else 2))   # kv head 0's query heads
+    got = _attend(gpu_device, kind, infinite)
+    seen = torch.zeros_like(clean, dtype=torch.bool)
+    seen[at:, mine, 5] = True
+    assert got[seen].isinf().all()
+    assert ((got - clean).abs()[~seen] <= bar).all()
+    got = _attend(gpu_device, kind, nan_key)
+    assert got[rows >= at][:, mine].isnan().all()
+    seen = torch.zeros_like(clean, dtype=torch.bool)
+    seen[at:, mine] = True
+    assert ((got - clean).abs()[~seen] <= bar).all()
 
 
 @pytest.mark.gpu

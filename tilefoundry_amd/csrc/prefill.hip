@@ -546,8 +546,8 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_pa
   float mx[CT], sum[CT], self[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    mx[ct] = self[ct] = kPanelNegInf;
-    sum[ct] = 0.f;
+    mx[ct] = kPanelNegInf;
+    self[ct] = sum[ct] = 0.f;                // self: the own key's lane of a column's four
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[dt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -667,6 +667,85 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_pa
     __syncthreads();
   }
 
+  // A product takes every position of a tile into every row: an infinite or NaN value
+  // past a row reaches it as 0 * inf, and the parts of a split infinite value cancel.
+  // Either leaves a NaN, so a wave that holds one takes its columns again position by
+  // position, each from its own past alone, as a step's lanes do.
+  float probe = 0.f;
+#pragma unroll
+  for (int ct = 0; ct < CT; ++ct) {
+    probe = fmaf(sum[ct], 0.f, probe);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) probe = fmaf(o[dt][ct][e], 0.f, probe);
+  }
+  if (__any(probe != 0.f)) {
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+      const int c = 16 * (CT * wave + ct) + r;
+      const int64_t q0 =
+          ((int64_t)(tl.row0 + min(c % QT, tl.rows - 1)) * heads + h * G + c / QT) * D + 8 * kq;
+      // the score of position p, the same in a column's four lanes
+      auto score_of = [&](int p) {
+        const bf16* kp =
+            kpool + (((int64_t)page_at(p / kPage) * kv_heads + h) * kPage + p % kPage) * D + 8 * kq;
+        float a = 0.f, lo, hi;
+#pragma unroll 1
+        for (int s = 0; s < DS; ++s) {
+          const u32x4 w = load16(kp + 32 * s);
+          if constexpr (kPol == kAttnF32) {
+            const f32x4* qp = reinterpret_cast<const f32x4*>((const float*)q_in + q0 + 32 * s);
+            const f32x4 x = qp[0], y = qp[1];
+            a = fmaf(x.x, bf_lo(w.x), fmaf(x.y, bf_hi(w.x), a));
+            a = fmaf(x.z, bf_lo(w.y), fmaf(x.w, bf_hi(w.y), a));
+            a = fmaf(y.x, bf_lo(w.z), fmaf(y.y, bf_hi(w.z), a));
+            a = fmaf(y.z, bf_lo(w.w), fmaf(y.w, bf_hi(w.w), a));
+          } else {
+            a = dot8(w, load16((const bf16*)q_in + q0 + 32 * s), a);
+          }
+        }
+        pair16(a, lo, hi);
+        a = lo + hi;
+        pair32(a, lo, hi);
+        a = lo + hi;
+        if (kPol == kAttnF32) return p == qpos[ct] ? own[ct] : a;
+        return kPol == kAttnDense ? rbf(a) : rbf(a) * scale;
+      };
+      float m = kPanelNegInf, l = 0.f, sn = 0.f;
+#pragma unroll 1
+      for (int p = 0; p <= last; ++p) {
+        const float s = score_of(p);
+        if (p <= qpos[ct]) m = fmaxf(m, s);
+        if (p == qpos[ct]) sn = s;
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int p = 0; p <= last; ++p) {
+        const float x = score_of(p) - m;
+        if (p >= qpos[ct] + (kPol == kAttnDense ? 0 : 1)) continue;
+        float w = expf(kPol == kAttnDense ? rbf(x) : x);
+        if (kPol == kAttnDense) w = rbf(w);
+        l += w;
+        if (kPol == kAttnGranite) w = rbf(w);
+        const bf16* vp = vpool +
+            (((int64_t)page_at(p / kPage) * kv_heads + h) * kPage + p % kPage) * D + 4 * kq;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+          const u32x2 vw = *reinterpret_cast<const u32x2*>(vp + 16 * dt);
+          o[dt][ct].x = fmaf(w, bf_lo(vw.x), o[dt][ct].x);
+          o[dt][ct].y = fmaf(w, bf_hi(vw.x), o[dt][ct].y);
+          o[dt][ct].z = fmaf(w, bf_lo(vw.y), o[dt][ct].z);
+          o[dt][ct].w = fmaf(w, bf_hi(vw.y), o[dt][ct].w);
+        }
+      }
+      mx[ct] = m;
+      sum[ct] = kq == 0 ? l : 0.f;
+      self[ct] = kq == 0 ? sn : 0.f;
+    }
+  }
+
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int c = 16 * (CT * wave + ct) + r;
@@ -675,10 +754,10 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_pa
     l = lo + hi;
     pair32(l, lo, hi);
     l = lo + hi;
-    pair16(sn, lo, hi);
-    sn = fmaxf(lo, hi);
+    pair16(sn, lo, hi);                      // (a NaN of the own key stays one)
+    sn = lo + hi;
     pair32(sn, lo, hi);
-    sn = fmaxf(lo, hi);
+    sn = lo + hi;
     const float pn = rbf(expf(rbf(sn - mx[ct])));
     const float inv = 1.f / (kPol == kAttnDense ? rbf(rbf(l) + pn) : l);
     const int P = qpos[ct];

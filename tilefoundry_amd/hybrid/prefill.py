@@ -8,8 +8,7 @@ and experts for all rows together, attention over the paged cache, and only the
 recurrence token by token, its state in registers.  Each row is valued as a step at
 its position values it, with f32 sums in other orders, and Granite's attention takes
 exact products and rounds each probability against the maximum so far (a step rounds
-the products and the normalised probabilities).  An infinite value in the cache reaches
-the rows of its 64-position tile that precede it; finite ones reach only later rows.
+the products and the normalised probabilities).
 
 The pass leaves what the walk leaves for the next step: caches, recurrent states and
 convolution windows of positions 0 .. n - 2.  So the last layer stops at its mixer's
