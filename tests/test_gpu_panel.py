@@ -257,6 +257,31 @@ def test_panel_attn_rows_do_not_see_what_follows_them(gpu_device, kind, at):
 
 
 @pytest.mark.gpu
+def test_panel_attn_probabilities_are_exactly_rounded(gpu_device):
+    """p = bf16(exp(x)) for every bf16 x in (-87, 0] (its result a normal number): one
+    sequence per x, a past key that scores x beside the row's own, which scores 0.  The
+    output p * 1 / bf16(p + 1), taken in f32 and rounded, is equal to the bit."""
+    L = _lib.lib()
+    x = torch.arange(0x8000, 0xc2ae, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    n, D, bf = len(x), 64, torch.bfloat16
+    z = lambda *shape, dtype=bf: torch.zeros(*shape, device=gpu_device, dtype=dtype)
+    q, k, v = z(n, 2, D), z(n, 1, 16, D), z(n, 1, 16, D)
+    q[:, :, 0], k[:, 0, 0, 0], v[:, 0, 0, 0] = 1, x.to(gpu_device), 1
+    i = torch.arange(n, dtype=torch.int32, device=gpu_device)
+    tiles = torch.stack((i, torch.ones_like(i), i, torch.ones_like(i)), 1).contiguous()
+    out, err = z(-(-n // 32) * 32 * 2 * D), z(1, dtype=torch.int32)
+    L.tfd_panel_attn(q.data_ptr(), tiles.data_ptr(), n, 2, 1, D, i.data_ptr(), 1, k.data_ptr(),
+                     v.data_ptr(), n, out.data_ptr(), err.data_ptr(),
+                     torch.cuda.current_stream().cuda_stream)
+    got = unpanel(out, n, 2 * D).view(n, 2, D)[:, :, 0].cpu()
+    assert int(err.item()) == 0
+    p = torch.exp(x.double()).to(bf).float()
+    want = (p * (1 / (p + 1).to(bf).float())).to(bf)
+    off = (got != want[:, None]).sum()
+    assert off == 0, (int(off), x[(got != want[:, None]).any(1)][:8].tolist())
+
+
+@pytest.mark.gpu
 def test_passes_cut_anywhere_fill_the_same_cache(gpu_device, monkeypatch):
     """Three prompts in one pass and in passes of 64 rows: the same caches to the
     bf16 bar (other GEMM shapes, other f32 orders)."""

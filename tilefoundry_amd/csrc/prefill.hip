@@ -394,9 +394,11 @@ struct PanelTile {
   int row0, rows, seq, pos0;
 };
 
-// exp(x) for x <= 0 where the result is rounded to bf16 or summed beside values that
-// are: 2^(x log2 e) on the transcendental unit, off by at most |x| 2^-24 + 2^-22 of the
-// value (below 2^-17 wherever the value is above 2^-40), against 2^-9 of the rounding.
+// bf16(exp(x)) for bf16 x <= 0, before its rounding: 2^(x log2 e) on the transcendental
+// unit, off by at most |x| 2^-24 + 2^-22 of the value.  Rounded to bf16 it is the correctly
+// rounded exp(x) for every bf16 x whose result is a normal number, as expf's is
+// (test_panel_attn_probabilities_are_exactly_rounded takes all 17,070 of them); where the
+// value itself is summed in f32 it would not be, and those policies call expf.
 __device__ __forceinline__ float exp_for_bf16(float x) {
   return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f);
 }
@@ -634,8 +636,7 @@ __global__ __launch_bounds__(kBlock, D <= 128 ? (CT == 1 ? 3 : 2) : 1) void k_pa
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const float x = st[2 * kk + p][ct][e] - m1;
-            pe[p][e] = kPol == kAttnDense ? exp_for_bf16(rbf(x)) :
-                       kPol == kAttnGranite ? exp_for_bf16(x) : expf(x);
+            pe[p][e] = kPol == kAttnDense ? exp_for_bf16(rbf(x)) : expf(x);
             if (kPol != kAttnDense) sum[ct] += pe[p][e];
           }
         if constexpr (kPol == kAttnF32) {
