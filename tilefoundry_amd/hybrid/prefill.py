@@ -62,7 +62,8 @@ class _Pass:
     def _reserve(self, M):
         if M <= self.rows:
             return
-        R = self.rows = -(-M // 32) * 32
+        R = -(-M // 32) * 32
+        self.rows = 0                       # until every buffer below holds R rows
         c, H, k = self.cfg, self.H, self.k
         shapes = [(H, self.in_rows), (self.out_k, H), (H, c.experts), (H, 2 * c.shared_inter),
                   (c.shared_inter, H)]
@@ -84,6 +85,7 @@ class _Pass:
         self.moe_hidden, self.d = z(R * k, c.moe_inter), z(R * k, H)
         self.shared = z(R * c.shared_inter)
         self._mixer_buffers(R, z)
+        self.rows = R
 
     # ------------------------------------------------------------------ pieces
     def _gemm(self, x, w, scale, M, K, N, s):

@@ -158,7 +158,8 @@ class Prefill:
         """Workspaces for passes of up to M rows."""
         if M <= self.rows:
             return
-        R = self.rows = -(-M // 32) * 32
+        R = -(-M // 32) * 32
+        self.rows = 0                       # until every buffer below holds R rows
         dev, bf, f32 = self.dev, torch.bfloat16, torch.float32
         shapes = [(self.H, self.qkv_n), (self.QD, self.H), (self.I, self.H), (self.H, 2 * self.I)]
         part = 1
@@ -174,6 +175,7 @@ class Prefill:
         self.attn = torch.zeros(R * self.QD, device=dev, dtype=bf)
         self.hmid = torch.zeros(R * self.I, device=dev, dtype=bf)
         self.part = torch.empty(part, device=dev, dtype=f32)
+        self.rows = R
 
     def _gemm(self, x, w, M, K, N, s):
         """K-split partial sums of x @ w^T -> their number."""
