@@ -6,7 +6,9 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from tilefoundry_amd.hybrid import prefill as hybrid
 from tilefoundry_amd.hybrid.prefill import GranitePass, Qwen35Pass
+from tilefoundry_amd.qwen3 import prefill as qwen3
 from tilefoundry_amd.qwen3.prefill import Prefill
 
 LIB = SimpleNamespace(tfd_panel_gemm_slices=lambda M, K, N: 2)
@@ -46,9 +48,22 @@ def _hybrid(cls):
     return p, sizes
 
 
-@pytest.mark.parametrize("make", [_qwen3, lambda: _hybrid(Qwen35Pass),
-                                  lambda: _hybrid(GranitePass)], ids=["qwen3", "qwen3_5", "granite"])
-def test_a_failed_growth_promises_nothing(monkeypatch, make):
+PASSES = pytest.mark.parametrize("make", [_qwen3, lambda: _hybrid(Qwen35Pass),
+                                          lambda: _hybrid(GranitePass)],
+                                 ids=["qwen3", "qwen3_5", "granite"])
+
+
+@pytest.fixture
+def waits(monkeypatch):
+    """Called in the place of a wait for the device's current stream."""
+    calls = []
+    for m in (qwen3, hybrid):
+        monkeypatch.setattr(m, "wait_for_work", lambda device: [f() for f in calls])
+    return calls
+
+
+@PASSES
+def test_a_failed_growth_promises_nothing(monkeypatch, waits, make):
     """Growing fails at each of its allocations in turn (out of memory, caught by the
     caller): the next pass of the larger size still finds every buffer large enough."""
     real = {n: getattr(torch, n) for n in ("empty", "zeros")}
@@ -80,3 +95,19 @@ def test_a_failed_growth_promises_nothing(monkeypatch, make):
         else:
             break
     assert fails_at > 5
+
+
+@PASSES
+def test_buffers_in_use_go_after_a_wait(waits, make):
+    """Growing drops buffers that a pass on this stream may still read: it waits once,
+    with all of them in place; a first pass and one that fits wait for nothing."""
+    p, sizes = make()
+    seen = []
+    waits.append(lambda: seen.append({n: getattr(p, n).data_ptr() for n in before}))
+    before = {}
+    p._reserve(32)
+    p._reserve(17)
+    assert not seen
+    before = {n: getattr(p, n).data_ptr() for n in sizes(32)}
+    p._reserve(96)
+    assert seen == [before]

@@ -24,7 +24,7 @@ import torch
 
 from .. import _lib
 from .._lib import lib, ptr
-from ..qwen3.prefill import plan_passes, token_array
+from ..qwen3.prefill import plan_passes, token_array, wait_for_work
 
 MAX_PASS = 1024             # rows of one pass: its workspaces take up to about 0.4 GB
 
@@ -63,6 +63,8 @@ class _Pass:
         if M <= self.rows:
             return
         R = -(-M // 32) * 32
+        if self.rows:
+            wait_for_work(self.dev)
         self.rows = 0                       # until every buffer below holds R rows
         c, H, k = self.cfg, self.H, self.k
         shapes = [(H, self.in_rows), (self.out_k, H), (H, c.experts), (H, 2 * c.shared_inter),

@@ -66,6 +66,13 @@ def int32_ids(tokens) -> np.ndarray:
     return ids.astype(np.int32)
 
 
+def wait_for_work(device):
+    """Wait for the current stream, before buffers go that launches on it may still use:
+    the allocator hands a freed block on at once to the stream that allocated it, which
+    need not be this one."""
+    torch.cuda.current_stream(device).synchronize()
+
+
 def in_vocab(tokens: np.ndarray, vocab: int) -> bool:
     return tokens.size == 0 or (int(tokens.min()) >= 0 and int(tokens.max()) < vocab)
 
@@ -159,6 +166,8 @@ class Prefill:
         if M <= self.rows:
             return
         R = -(-M // 32) * 32
+        if self.rows:
+            wait_for_work(self.dev)
         self.rows = 0                       # until every buffer below holds R rows
         dev, bf, f32 = self.dev, torch.bfloat16, torch.float32
         shapes = [(self.H, self.qkv_n), (self.QD, self.H), (self.I, self.H), (self.H, 2 * self.I)]
