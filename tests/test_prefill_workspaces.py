@@ -1,6 +1,8 @@
-"""The workspaces of prompt passes (qwen3/prefill.py, hybrid/prefill.py) on the CPU:
-kernels take them as raw pointers with the pass's rows, so a pass must never find
-buffers of fewer rows than it was promised."""
+"""The host side of prompt passes (qwen3/prefill.py, hybrid/prefill.py) on the CPU.
+
+Workspaces: kernels take them as raw pointers with the pass's rows, so a pass must
+never find buffers of fewer rows than it was promised.  Dispatch: which prompts of the
+hybrids go through a pass and which through the decode step."""
 from types import SimpleNamespace
 
 import pytest
@@ -111,3 +113,30 @@ def test_buffers_in_use_go_after_a_wait(waits, make):
     before = {n: getattr(p, n).data_ptr() for n in sizes(32)}
     p._reserve(96)
     assert seen == [before]
+
+
+def _prefilled(monkeypatch, cls, rows, n):
+    """A prefill of *rows* prompts of *n* tokens on an engine whose sizes a pass takes ->
+    (positions walked, whether a pass object was built)."""
+    walked, built = [], []
+    monkeypatch.setattr(cls, "__init__", lambda self, eng: built.append(eng))
+    monkeypatch.setattr(cls, "takes", staticmethod(lambda eng: True))
+    monkeypatch.setattr(cls, "run", lambda self, prompts: None)
+    monkeypatch.setattr(hybrid, "ptr", lambda t: None)
+    z = torch.zeros(rows, dtype=torch.int64)
+    eng = SimpleNamespace(B=rows, nsteps=16, replay=lambda: walked.append(1), pos=z.clone(),
+                          ids=z.clone(), embed=z, emb=z, err=z, _stream=lambda: 0,
+                          cfg=SimpleNamespace(hidden=8, vocab=16), routes=None,
+                          _load_prompts=lambda prompts: None,
+                          _lib=SimpleNamespace(tfd_embed_rows_bf16=lambda *a: None))
+    hybrid.prefill(eng, cls, [list(range(1, n + 1)) for _ in range(rows)])
+    return len(walked), bool(built)
+
+
+@pytest.mark.parametrize("cls", [Qwen35Pass, GranitePass])
+@pytest.mark.parametrize("rows", [1, 2, 16])
+def test_a_walked_prompt_builds_no_pass(monkeypatch, cls, rows):
+    """One position is walked: nothing is packed or kept for it."""
+    assert _prefilled(monkeypatch, cls, rows, 1) == (0, False)
+    assert _prefilled(monkeypatch, cls, rows, 2) == (1, False)
+    assert _prefilled(monkeypatch, cls, rows, 4) == (0, True)

@@ -42,6 +42,11 @@ class _Pass:
     policy: int
     fp8: bool
 
+    @staticmethod
+    def step_positions(seqs: int) -> int:
+        """Positions per sequence up to which the decode step's walk is as fast."""
+        return 1
+
     def __init__(self, eng):
         # the engine holds this pass: a strong reference back would keep both, and
         # their device memory, until a garbage collection
@@ -338,20 +343,15 @@ def prefill(eng, passes, prompts: list[list[int]]):
     if n > eng.nsteps:
         raise ValueError(f"prompt {n} exceeds {eng.nsteps} steps")
     eng._load_prompts(prompts)
-    if n == 1:
-        return
-    if not passes.takes(eng):
+    # One position: a step's kernels, made for a row a sequence, are faster than a pass
+    # (four layers, one sequence: Qwen3.5 319 against 577 us, Granite 449 / 628; two
+    # positions 813 / 648 in Granite, 547 / 584 in Qwen3.5: ``step_positions``).
+    if n - 1 <= passes.step_positions(eng.B) or not passes.takes(eng):
         for _ in range(n - 1):
             eng.replay()
         return
     if getattr(eng, "_prefiller", None) is None:
         eng._prefiller = passes(eng)
-    if n == 2:
-        # one position: a step's kernels, made for a row a sequence, are faster than a
-        # pass (four layers, one sequence: Qwen3.5 319 against 577 us, Granite 449 / 628;
-        # two positions 547 / 584 and 813 / 648, eight 1,901 / 676 and 2,936 / 793)
-        eng.replay()
-        return
     eng._prefiller.run(prompts)
     eng.pos.fill_(n - 1)
     eng.ids.copy_(torch.tensor([p[-1] for p in prompts], dtype=torch.int64))
