@@ -140,3 +140,10 @@ def test_a_walked_prompt_builds_no_pass(monkeypatch, cls, rows):
     assert _prefilled(monkeypatch, cls, rows, 1) == (0, False)
     assert _prefilled(monkeypatch, cls, rows, 2) == (1, False)
     assert _prefilled(monkeypatch, cls, rows, 4) == (0, True)
+
+
+def test_two_positions_of_one_qwen3_5_sequence_are_walked(monkeypatch):
+    """A pass over them is slower than two steps; Granite's, and more sequences', is not."""
+    assert _prefilled(monkeypatch, Qwen35Pass, 1, 3) == (2, False)
+    assert _prefilled(monkeypatch, Qwen35Pass, 2, 3) == (0, True)
+    assert _prefilled(monkeypatch, GranitePass, 1, 3) == (0, True)

@@ -208,6 +208,12 @@ class Qwen35Pass(_Pass):
         super().__init__(eng)
 
     @staticmethod
+    def step_positions(seqs: int) -> int:
+        # four layers: one sequence's two positions 604 us walked, 691 in a pass, three
+        # 829 / 682; two sequences' two positions 774 / 722, sixteen's 1,886 / 1,587
+        return 2 if seqs == 1 else 1
+
+    @staticmethod
     def takes(eng) -> bool:
         """Whether the kernels of a pass cover this engine's sizes."""
         c = eng.cfg
@@ -345,7 +351,7 @@ def prefill(eng, passes, prompts: list[list[int]]):
     eng._load_prompts(prompts)
     # One position: a step's kernels, made for a row a sequence, are faster than a pass
     # (four layers, one sequence: Qwen3.5 319 against 577 us, Granite 449 / 628; two
-    # positions 813 / 648 in Granite, 547 / 584 in Qwen3.5: ``step_positions``).
+    # positions of Granite 813 / 648; of Qwen3.5 see its ``step_positions``).
     if n - 1 <= passes.step_positions(eng.B) or not passes.takes(eng):
         for _ in range(n - 1):
             eng.replay()
