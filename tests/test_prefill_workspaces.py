@@ -115,7 +115,7 @@ def test_buffers_in_use_go_after_a_wait(waits, make):
     assert seen == [before]
 
 
-def _prefilled(monkeypatch, cls, rows, n):
+def _prefilled(monkeypatch, cls, rows, n, routes=None):
     """A prefill of *rows* prompts of *n* tokens on an engine whose sizes a pass takes ->
     (positions walked, whether a pass object was built)."""
     walked, built = [], []
@@ -126,7 +126,7 @@ def _prefilled(monkeypatch, cls, rows, n):
     z = torch.zeros(rows, dtype=torch.int64)
     eng = SimpleNamespace(B=rows, nsteps=16, replay=lambda: walked.append(1), pos=z.clone(),
                           ids=z.clone(), embed=z, emb=z, err=z, _stream=lambda: 0,
-                          cfg=SimpleNamespace(hidden=8, vocab=16), routes=None,
+                          cfg=SimpleNamespace(hidden=8, vocab=16), routes=routes,
                           _load_prompts=lambda prompts: None,
                           _lib=SimpleNamespace(tfd_embed_rows_bf16=lambda *a: None))
     hybrid.prefill(eng, cls, [list(range(1, n + 1)) for _ in range(rows)])
@@ -147,3 +147,10 @@ def test_two_positions_of_one_qwen3_5_sequence_are_walked(monkeypatch):
     assert _prefilled(monkeypatch, Qwen35Pass, 1, 3) == (2, False)
     assert _prefilled(monkeypatch, Qwen35Pass, 2, 3) == (0, True)
     assert _prefilled(monkeypatch, GranitePass, 1, 3) == (0, True)
+
+
+@pytest.mark.parametrize("cls", [Qwen35Pass, GranitePass])
+def test_an_engine_that_records_routes_is_walked(monkeypatch, cls):
+    """``record_routes`` engines hold the experts of the last position walked: a pass has
+    none to leave."""
+    assert _prefilled(monkeypatch, cls, 2, 9, routes=torch.zeros(1)) == (8, False)

@@ -339,7 +339,8 @@ class GranitePass(_Pass):
 
 def prefill(eng, passes, prompts: list[list[int]]):
     """Bring *eng* to every prompt's last token: passes of class *passes* where their
-    kernels take the engine's sizes, else the decode step walked position by position."""
+    kernels take the engine's sizes, else the decode step walked position by position.
+    (A pass leaves no routing and no logits of the prompt's own positions.)"""
     if len(prompts) != eng.B or any(len(p) < 1 for p in prompts):
         raise ValueError(f"need {eng.B} non-empty prompts")
     if len({len(p) for p in prompts}) != 1:
@@ -352,7 +353,9 @@ def prefill(eng, passes, prompts: list[list[int]]):
     # One position: a step's kernels, made for a row a sequence, are faster than a pass
     # (four layers, one sequence: Qwen3.5 319 against 577 us, Granite 449 / 628; two
     # positions of Granite 813 / 648; of Qwen3.5 see its ``step_positions``).
-    if n - 1 <= passes.step_positions(eng.B) or not passes.takes(eng):
+    # An engine that records its routing keeps the last walked position's.
+    walk = n - 1 <= passes.step_positions(eng.B) or eng.routes is not None
+    if walk or not passes.takes(eng):
         for _ in range(n - 1):
             eng.replay()
         return
