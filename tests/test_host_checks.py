@@ -95,3 +95,11 @@ def test_hybrid_validate_rejects_what_the_kernels_cannot_read(model):
     retyped[victim] = w[victim].to(torch.float16)
     with pytest.raises(ValueError, match="dtype"):
         mod.validate(cfg, retyped)
+
+
+@pytest.mark.parametrize("M,K,N", [(0, 256, 64), (32, 128, 64), (32, 256, 0), (32, 256, 42)])
+def test_panel_gemm_slices_of_a_refused_shape_are_zero(M, K, N):
+    """What tfd_panel_gemm_bf16 refuses has no slices to size a buffer for."""
+    from tilefoundry_amd._lib import lib
+
+    assert lib().tfd_panel_gemm_slices(M, K, N) == 0

@@ -917,7 +917,7 @@ PanelPlan panel_plan(int M, int K, int N) {
 extern "C" {
 
 int tfd_panel_gemm_slices(int M, int K, int N) {
-  if (M <= 0 || K <= 0 || K % 256 || N <= 0) return 0;
+  if (M <= 0 || K <= 0 || K % 256 || N <= 0 || N % 4) return 0;
   return panel_plan(M, K, N).slices;
 }
 
