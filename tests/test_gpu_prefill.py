@@ -150,3 +150,26 @@ def test_batch_prefill_then_greedy_matches_the_oracle(gpu_device):
                            strict=False)
             print(f"sequence {b} ({len(p)}-token prompt), {name}: identical to the oracle for "
                   f"{32 if k is None else k} of 32 steps", flush=True)
+
+
+@pytest.mark.parametrize("cls", [Engine, BatchEngine])
+def test_an_engine_that_prefilled_is_freed_when_dropped(gpu_device, cls):
+    """The engine and its pass hold no cycle: their device memory goes with the last
+    reference, not with a later garbage collection."""
+    import gc
+    import weakref
+
+    w = synthetic_weights(SMALL, seed=1, norms="ones")
+    prompt = _prompt(9, SMALL.vocab_size, seed=1)
+    batched = cls is BatchEngine
+    eng = cls(SMALL, w, device=gpu_device, max_new=8, prompt_room=16,
+              **({"batch": 1} if batched else {}))
+    gc.collect()
+    gc.disable()
+    try:
+        eng.prefill([prompt] if batched else prompt)
+        gone = weakref.ref(eng)
+        del eng
+        assert gone() is None
+    finally:
+        gc.enable()

@@ -17,6 +17,7 @@ The batch-1 engine's structure (``engine.py``; the reference's
 """
 from __future__ import annotations
 
+import weakref
 from time import perf_counter
 
 import numpy as np
@@ -337,7 +338,7 @@ class BatchEngine:
         if len(prompts) != self.B or any(len(p) < 1 for p in prompts):
             raise ValueError(f"need {self.B} non-empty prompts")
         if getattr(self, "_prefiller", None) is None:
-            self._prefiller = Prefill(self, packed=True)
+            self._prefiller = Prefill(weakref.proxy(self), packed=True)
         self._load_prompts(prompts)
         self._prefiller.run_many([(p[:-1], 0, b) for b, p in enumerate(prompts) if len(p) > 1])
         self.pos.copy_(torch.tensor([len(p) - 1 for p in prompts], dtype=torch.int32))

@@ -21,6 +21,7 @@ What differs, MI355X-first:
 from __future__ import annotations
 
 import ctypes
+import weakref
 from dataclasses import dataclass
 from time import perf_counter
 
@@ -383,7 +384,7 @@ class Engine:
         if pl < 2:
             return
         if getattr(self, "_prefiller", None) is None:
-            self._prefiller = Prefill(self)
+            self._prefiller = Prefill(weakref.proxy(self))    # no cycle: see its docstring
         self._prefiller.run(prompt_ids[:-1], 0)
         self.pos.fill_(pl - 1)
         self.ids.fill_(int(prompt_ids[-1]))

@@ -125,7 +125,9 @@ class Prefill:
     pool), ``cos``/``sin``, ``cap``).  With *packed* False the projections are
     re-laid once into the skinny GEMMs' operand blocks (one more copy of the
     layer weights in HBM); a batch engine's layers are already in that order.
-    Workspaces grow to the largest pass seen, ``MAX_PASS`` rows at most."""
+    An engine that keeps its own pass hands in a weak proxy of itself: with a cycle the
+    device memory of both would stay until a garbage collection.  Workspaces grow to the
+    largest pass seen, ``MAX_PASS`` rows at most."""
 
     def __init__(self, engine, packed: bool = False):
         e = engine
