@@ -206,9 +206,9 @@ def cpu_baseline(weights, prompt, budget_s: float) -> dict:
 
 def bench_c3(args) -> int:
     """Workload C3: the same model at batch 32, every sequence with a
-    4096-token random context (built untimed: by default prefilled one
-    sequence at a time, 32 positions per pass; `--c3-context walk` walks the
-    contexts with batched decode steps instead), then `--steps` (default 256)
+    4096-token random context (built untimed: by default prefilled in passes of
+    up to 4,096 positions, `--c3-context walk` walks the contexts with batched
+    decode steps instead), then `--steps` (default 256)
     timed steps of 32 tokens each."""
     import torch
 

@@ -53,12 +53,15 @@ def _left(eng):
     return out
 
 
-# one row a sequence (windows reach back past the pass), fewer than three, whole scan
-# chunks and one more, passes cut in the middle, expert tiles of 64 rows and a rest
+# no pass at all (one position is the walk's own step); two rows a sequence (fewer than
+# a window); whole scan chunks and one more; passes cut in the middle, the last of two
+# rows a sequence or of one (its window reaches back past the pass); expert tiles of 64
+# rows and a rest
 @pytest.mark.gpu
 @pytest.mark.parametrize("model", ["qwen3_5", "granite"])
 @pytest.mark.parametrize("rows,n,most", [(1, 2, 1024), (3, 3, 1024), (1, 18, 1024), (5, 40, 1024),
-                                         (2, 99, 64), (3, 66, 1024)])
+                                         (2, 99, 64), (3, 66, 1024), (2, 98, 64),
+                                         (1, 66, 64)])
 def test_pass_is_the_walk(gpu_device, monkeypatch, model, rows, n, most):
     monkeypatch.setattr(P, "MAX_PASS", most)
     eng = _engine(model, rows, gpu_device, n + 8)

@@ -119,7 +119,8 @@ def test_panel_add_norm(gpu_device, slices, M, n):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("D,G", [(128, 2), (64, 2), (128, 1)])
-@pytest.mark.parametrize("segs", [[(0, 1)], [(0, 64), (63, 1)], [(0, 200), (70, 129), (128, 3)]])
+@pytest.mark.parametrize("segs", [[(0, 1)], [(0, 64), (63, 1)], [(0, 200), (70, 129), (128, 3)],
+                                  [(2900, 301), (0, 700)]])
 def test_panel_attn(gpu_device, D, G, segs):
     """(first position, rows) segments over filled pages against f32 softmax.  Scores
     are rounded to bf16 (|s| < 8 here: 2^-6 absolute), probabilities twice and the
@@ -304,6 +305,58 @@ def test_passes_cut_anywhere_fill_the_same_cache(gpu_device, monkeypatch):
     eng.check_errors()
     assert_close_bf16(eng.kpool, k, max_rel=2e-2, name="k")
     assert_close_bf16(eng.vpool, v, max_rel=2e-2, name="v")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+def test_panel_moe_with_uneven_picks(gpu_device, fp8):
+    """Experts picked by none, 1, 63, 64, 65 and 207 of 200 rows (two slots each): every
+    entry's two projections against f64 sums.  hidden is rounded twice more before its
+    own rounding (gate, up; 2^-9 each), the output once: 2^-6 of the output's norm."""
+    L = _lib.lib()
+    s = torch.cuda.current_stream().cuda_stream
+    M, k, E, H, I = 200, 2, 7, 512, 256
+    g = torch.Generator(device=gpu_device).manual_seed(5 + fp8)
+    counts = [0, 1, 63, 64, 65, 207, 0]
+    picks = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    idx = picks[torch.randperm(M * k, generator=torch.Generator().manual_seed(2))].view(M, k)
+    rn = lambda *shape: torch.randn(*shape, generator=g, device=gpu_device)
+    x = rn(M, H).to(torch.bfloat16)
+    a = _lib.TfdPanelMoeArgs()
+    keep, mats = [], {}
+    for name, rows, cols in (("gate", I, H), ("up", I, H), ("down", H, I)):
+        w = rn(E * rows, cols)
+        if fp8:
+            w8 = w.to(torch.float8_e4m3fn)
+            sc = torch.rand(E * rows, generator=g, device=gpu_device) * 0.05 + 0.05
+            packed = torch.empty(E * rows * cols, dtype=torch.uint8, device=gpu_device)
+            L.tfd_pack_skinny_fp8(w8.data_ptr(), cols, E * rows, cols, packed.data_ptr(), s)
+            keep += [w8, sc, packed]
+            setattr(a, f"w_{name}", packed.data_ptr())
+            setattr(a, f"s_{name}", sc.data_ptr())
+            mats[name] = (w8.double() * sc.double()[:, None]).view(E, rows, cols)
+        else:
+            w = (0.08 * w).to(torch.bfloat16)
+            keep.append(w)
+            setattr(a, f"w_{name}", w.data_ptr())
+            mats[name] = w.double().view(E, rows, cols)
+    z = lambda n, dtype=torch.bfloat16: torch.zeros(n, dtype=dtype, device=gpu_device)
+    idxd = idx.to(torch.int32).to(gpu_device)
+    hidden, d, err = z(M * k * I), z(M * k * H), z(1, torch.int32)
+    groups = z(_lib.panel_moe_words(E, M * k), torch.int32)
+    a.x, a.idx, a.groups, a.hidden, a.d = (t.data_ptr() for t in (x, idxd, groups, hidden, d))
+    a.M, a.k, a.experts, a.H, a.I, a.fp8 = M, k, E, H, I, int(fp8)
+    a.policy, a.err = _lib.POLICY_BF16 if fp8 else _lib.POLICY_F32, err.data_ptr()
+    L.tfd_panel_moe(ctypes.addressof(a), s)
+    got = d.view(M, k, H).double()
+    assert int(err.item()) == 0
+    xd = x.double()
+    for m in range(M):
+        for j in range(k):
+            e = int(idx[m, j])
+            h = torch.nn.functional.silu(mats["gate"][e] @ xd[m]) * (mats["up"][e] @ xd[m])
+            want = mats["down"][e] @ h
+            assert (got[m, j] - want).norm() <= 2.0 ** -6 * want.norm(), (m, j, e)
 
 
 def test_token_array_takes_what_a_prompt_may_be():

@@ -6,11 +6,12 @@
   rounding may land one bf16 ulp away.
 * Greedy decoding after prefill matches the oracle's walk of the prompt: 64
   identical tokens on the config-1 shape (prompts of 40 and 71 tokens: two and
-  three 32-row chunks; persistent and graph decoding), and the Qwen3-1.7B layer
+  three 32-row panels, one and two attention tiles' worth of positions; persistent and
+  graph decoding), and the Qwen3-1.7B layer
   shape at two layers with the engine's usual near-tie rule (persistent and
   XCD decoding).
-* The batch engine's prefill (one sequence at a time through its page-table row
-  of the shared pool): every sequence's cache equals its own oracle walk, and
+* The batch engine's prefill (all sequences in one pass, each through its page-table
+  row of the shared pool): every sequence's cache equals its own oracle walk, and
   the batched greedy continuation after prefill is each sequence's oracle
   continuation, prompts of different lengths (one of a single token) together.
 """
@@ -79,7 +80,7 @@ def test_prefill_then_greedy_64_matches_the_oracle(gpu_device, mode, n):
 
 @pytest.mark.parametrize("mode", ["persistent", "xcd"])
 def test_prefill_at_the_layer_shape(gpu_device, mode):
-    """Two layers of the Qwen3-1.7B shape, a 70-token prompt (three chunks): the
+    """Two layers of the Qwen3-1.7B shape, a 70-token prompt (three panels): the
     continuation tracks the oracle's walk as decoding does (logits within the
     bar, a divergence only at a near-tie the measured error explains), and the
     engine's own walk of the prompt gives the same logits to the bf16 bar until
@@ -110,9 +111,9 @@ def _batch_cache(eng, layer, b, n):
     return eng.kpool[layer][page, :, row].float().cpu(), eng.vpool[layer][page, :, row].float().cpu()
 
 
-# room 4,096: the prefill's score rows are an allocation of megabytes, whose
-# first row is sequence 0's at position 0 -- a split with no prior position,
-# which still prefetches its next tile's scores from inside that row
+# room 72: the longest prompt ends in the table's last pages; room 4,096: the tables go
+# on for hundreds of pages past every prompt, and the tiles of the first sequence (four
+# rows) read ahead past its end
 @pytest.mark.parametrize("room", [72, 4096])
 def test_batch_prefill_caches_match_the_oracle_walks(gpu_device, room):
     w = synthetic_weights(SMALL, seed=1, norms="random")
