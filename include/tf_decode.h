@@ -275,7 +275,8 @@ int tfd_embed_rows_bf16(const void* table, const int64_t* ids, void* out, int ld
  * (tests/fixtures/placed/qwen3_1_7b_pd.py:55-230). */
 #define TFD_PANEL_PARTIAL 0 /* out f32 [slices][M][N]: K-split partial sums */
 #define TFD_PANEL_SWIGLU 1  /* out panel order [M][N/2] (one slice only) */
-/* K slices tfd_panel_gemm_bf16 uses for a shape (0: a shape it does not take). */
+/* K slices tfd_panel_gemm_bf16 uses for a shape (0: one it does not take; whether
+ * TFD_PANEL_SWIGLU takes a one-slice shape is N/2 % 32 == 0 besides). */
 int tfd_panel_gemm_slices(int M, int K, int N);
 /* Y[m][n] = sum_k X[m][k] W[n][k], X in panel order, W packed by tfd_pack_skinny_bf16,
  * f32 sums; K % 256 == 0, N % 4 == 0.  TFD_PANEL_SWIGLU needs one slice and
@@ -302,7 +303,11 @@ int tfd_panel_attn_rows(int group);
 /* Causal attention of the rows over their sequences' pages (appended before the call).
  * tiles int32 [ntiles][4]: first row, rows (up to tfd_panel_attn_rows), sequence, the
  * first row's position; a tile's rows are consecutive positions.  out: panel order
- * [M][heads * head_dim].  (head_dim, group) of (128, 2), (64, 2) or (128, 1). */
+ * [M][heads * head_dim].  (head_dim, group) of (128, 2), (64, 2) or (128, 1).
+ * The decode entries round every product; here they are exact: s = bf16(q . k) and
+ * p = bf16(exp(bf16(s - m))) against the maximum m of the positions up to p's 64-position
+ * tile, p . v in f32.  A row reads its own position and those before it only, values that
+ * are not finite included.  Page-table entries past a tile's last row are not used. */
 int tfd_panel_attn(const void* q, const int32_t* tiles, int ntiles, int heads, int kv_heads,
                    int head_dim, const int32_t* page_table, int max_pages, const void* k_pool,
                    const void* v_pool, int num_pages, void* out, int32_t* err, void* stream);

@@ -445,7 +445,7 @@ int tfd_moe_experts_small(const TfdMoeArgs* args, void* stream);
  * Panel order and TFD_PANEL_PARTIAL sums as in tf_decode.h.  The reference walks its
  * prompts token by token (examples/qwen3_5_35b_a3b-tilelang/run.py,
  * examples/granite_4_0_h_small-cuda/run.py); each row is valued as a step at its
- * position values it, f32 summation orders apart. */
+ * position values it, f32 summation orders and tfd_panel_gqa's products apart. */
 
 /* tfd_panel_gemm_bf16 over tfd_pack_skinny_fp8 weights and their f32 row scales. */
 int tfd_panel_gemm_fp8(const void* x, const void* w, const float* scale, int M, int K, int N,
@@ -541,7 +541,13 @@ typedef struct {
 int tfd_panel_mamba(const TfdPanelMambaArgs* args, void* stream);
 
 /* A hybrid's attention layer over the rows, between its projections: append and causal
- * attention (tfd_gqa_decode's arithmetic per policy) -> panel order [M][heads * head_dim].
+ * attention -> panel order [M][heads * head_dim].  TFD_POLICY_F32: tfd_gqa_decode's
+ * arithmetic (f32 throughout; queries and probabilities as sums of three bf16 operands).
+ * TFD_POLICY_BF16: s = bf16(q . k) * scale with exact products (a step rounds each to
+ * bf16), p = exp(s - m) against the maximum m of the positions up to p's 64-position tile,
+ * summed in f32 and rounded to bf16 for p . v, the sum divided out at the end (a step
+ * rounds p / sum).  A row reads its own position and those before it only, values that are
+ * not finite included.
  * proj bf16 [M][ldp]; tiles as tfd_panel_attn's, of up to TFD_PANEL_GQA_ROWS_* rows.
  * Work: q (f32 for TFD_POLICY_F32, else bf16) [M][heads * head_dim]; TFD_POLICY_F32: gate
  * bf16 [M][heads * head_dim], self_scores f32 [M][heads]. */

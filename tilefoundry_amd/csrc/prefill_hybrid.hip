@@ -434,7 +434,8 @@ __global__ __launch_bounds__(kBlock) void k_pgdn_conv(TfdPanelGdnArgs a) {
 // eight lanes to a column, sixteen key rows each in registers; the tokens' q, k, v and
 // gates come through LDS, sixteen tokens at a time.
 // Bound: the chain of a token (64 multiply-adds a lane and two eight-lane sums): 250
-// tokens take 71 us, 0.28 us each; with the step's kernel a token's launch took 5.5.
+// tokens take 71 us, 0.28 us each; with the step's kernel a token's launch took 5.5.  One
+// sequence's 128 blocks (32 heads) leave half the compute units without one.
 constexpr int kScanT = 16;
 __global__ __launch_bounds__(kBlock) void k_pgdn_scan(TfdPanelGdnArgs a) {
   const int hv = blockIdx.y, b = blockIdx.z, tid = threadIdx.x;
@@ -570,7 +571,8 @@ __global__ __launch_bounds__(kBlock) void k_pmamba_conv(TfdPanelMambaArgs a) {
 // rows, eight lanes to a row, sixteen columns each in registers (columns 32 j + 4 ng
 // + e); bf16(dt B) and C come through LDS, sixteen tokens at a time and read a token
 // ahead.
-// Bound: the VALU, one wave to a SIMD (eleven operations a state and token with dt B
+// Bound: the VALU, one wave to a SIMD where a block runs: one sequence's 128 blocks (64
+// heads) leave half the compute units without one (eleven operations a state and token with dt B
 // formed by every row and one value to a conversion: 92 us for 190 tokens; six with two
 // values to a conversion and C's products summed in pairs: 71, 0.37 a token).
 __global__ __launch_bounds__(kBlock) void k_pmamba_scan(TfdPanelMambaArgs a) {

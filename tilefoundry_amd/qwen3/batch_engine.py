@@ -180,7 +180,7 @@ class BatchEngine:
         # f32 partial tiles of GEMMs that split K; 8 MiB covers every projection
         self.work = z(1 << 21, dtype=f32)
         # From nine rows on, the output and down projections leave K-split sums that the
-        # next norm adds (two launches for three, and no hand-off inside the GEMM).  A
+        # next norm adds (as many launches, and no hand-off inside the GEMM).  A
         # step of eight layers of Qwen3-1.7B: 578 against 648 us at 32 rows, 534 / 553
         # at 16, 518 / 520 at 8; at one row 503 / 464, where the skinny GEMM wastes less.
         self.panels = B > 8

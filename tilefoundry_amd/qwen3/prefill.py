@@ -10,7 +10,8 @@ sequences, through each layer (``csrc/prefill.hip``): every weight is read once 
 pass and every cached key once per 64 rows of a tile, where the decode kernels
 would read them once per 32 rows and once per row.  Each position is valued as a
 decode step at that position values it: the HIR's rounding points, with attention's
-products exact as the XCD kernel takes them, and other f32 summation orders.
+products exact as the XCD kernel takes them, each probability rounded against the
+maximum of the tiles so far, and other f32 summation orders.
 
 Prefill fills the cache for positions start .. start + n - 1 and leaves the
 hidden states of those rows unused: the last prompt token is then decoded as
