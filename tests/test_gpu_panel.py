@@ -379,6 +379,22 @@ def test_token_array_takes_what_a_prompt_may_be():
         int32_ids([(1 << 32) + 5])
 
 
+def test_token_array_takes_tensors_of_one_element():
+    """Ids as a sampling loop leaves them; text, rows and NaN are refused."""
+    import numpy as np
+
+    from tilefoundry_amd.qwen3.prefill import token_array
+
+    for p in ([torch.tensor([1]), torch.tensor([2])], [torch.tensor([1]), 2],
+              (torch.tensor([[1]]), torch.tensor(2)), torch.tensor([1, 2], dtype=torch.int32),
+              [1.0, 2.5], torch.tensor([1.0, 2.0]), [torch.tensor([1.5]), 2], np.array([1.0, 2.0])):
+        assert token_array(p).tolist() == [1, 2] and token_array(p).dtype == np.int64
+    for p in ("12", ["1", "2"], torch.tensor([[1], [2]]), np.array([[1], [2]]), [[1], [2]], 3,
+              [None], [torch.tensor([1, 2]), 3], [float("nan")], np.array([np.inf])):
+        with pytest.raises((ValueError, RuntimeError)):
+            token_array(p)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch", [8, 9, 17, 32])
 def test_batch_step_on_both_sides_of_nine_rows(gpu_device, batch):

@@ -24,6 +24,9 @@ go through together.
 """
 from __future__ import annotations
 
+from array import array
+from operator import index
+
 import numpy as np
 import torch
 
@@ -49,14 +52,25 @@ def attention_splits(rows: int, kv_heads: int, cap: int) -> int:
 def token_array(tokens) -> np.ndarray:
     """Token ids (any sequence of them) as an int64 array."""
     try:
-        ids = np.asarray(tokens, dtype=np.int64)
-    except TypeError:                       # values numpy cannot read, e.g. on a device
-        ids = np.array([int(t) for t in tokens], dtype=np.int64)
+        if isinstance(tokens, (list, tuple)):
+            try:                            # whole numbers, tensors of one element too
+                return np.array(array("q", tokens))
+            except TypeError:               # fractions are cut, as int() cuts them
+                return np.array([int(t) if isinstance(t, (float, np.floating, torch.Tensor))
+                                 else index(t) for t in tokens], dtype=np.int64)
+        if isinstance(tokens, torch.Tensor):
+            tokens = tokens.detach().cpu()
+            tokens = tokens.double() if tokens.is_floating_point() else tokens
+        ids = np.asarray(tokens)
+        if ids.ndim != 1 or ids.dtype.kind not in "biuf":
+            raise TypeError
     except OverflowError:
         raise ValueError("token ids must fit in 64 bits") from None
-    if ids.ndim != 1:
-        raise ValueError(f"token ids must be one sequence, got {ids.ndim} dimensions")
-    return ids
+    except TypeError:
+        raise ValueError("token ids must be one sequence of whole numbers") from None
+    if ids.dtype.kind == "f" and not (np.abs(ids) < 2.0 ** 63).all():
+        raise ValueError("token ids must fit in 64 bits")
+    return ids.astype(np.int64, copy=False)
 
 
 def int32_ids(tokens) -> np.ndarray:
