@@ -116,6 +116,21 @@ def test_skinny_gemm_within_one_ulp_of_exact(gpu_device, M, K, N, split):
         assert not work[:tiles].any()
 
 
+@pytest.mark.parametrize("M,K,N", [(16, 2560, 8448), (9, 1024, 8200), (1, 1280, 9000),
+                                   (16, 2048, 8192), (17, 2560, 8448), (4, 5120, 8192)])
+def test_skinny_gemm_writes_every_column_of_wide_shapes(gpu_device, M, K, N):
+    """512 tiles and more at up to 16 rows take two tiles a block where K is whole steps
+    of eight waves by eight, else one: every column is written, within one bf16 rounding
+    of the f64 sum and K 2^-24 sum |x w| of any f32 order."""
+    g = torch.Generator(device=gpu_device).manual_seed(K + N)
+    x = torch.randn(M, K, generator=g, device=gpu_device).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device=gpu_device) * 0.02).to(torch.bfloat16)
+    exact = x.double() @ w.double().t()
+    bound = exact.abs() * 2.0 ** -8 + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    got = _gemm(x, w, _lib.EPI_LOGITS, work=torch.zeros(1 << 21, device=gpu_device))
+    assert ((got.double() - exact.cpu()).abs() <= bound.cpu()).all()
+
+
 def test_pack_skinny_layout(gpu_device):
     """The packed layout, element by element: block (tile t, step s) is 1 KiB and
     lane l's 8 values are W[16t + l % 16][32s + 8(l // 16) + j]; padding rows are 0."""

@@ -818,12 +818,14 @@ SkinnyPlan skinny_plan(int K, int N, int64_t work_floats) {
 // (it needs no partials outside the block) and any K deeper than the LDS stage;
 // the X-stationary kernel takes the head, whose many tiles fill the chip and
 // whose X is worth keeping in LDS across them.  A block takes two tiles of a
-// wide shape when the batch is at most 16 rows (one X half per step), one
+// wide shape when the batch is at most 16 rows (one X half per step) and each of its
+// eight waves takes whole chunks of eight steps (the form two tiles are built in), one
 // otherwise (measured: M = 32 gate/up 1% faster per step with one, M = 1 and 16
 // about 1% slower).
 int ksplit_tiles(int M, int K, int N) {
   const int ntiles = (N + 15) / 16;
-  if (K > 2048 || ntiles < 4 * compute_units()) return ntiles >= 512 && M <= 16 ? 2 : 1;
+  if (K > 2048 || ntiles < 4 * compute_units())
+    return ntiles >= 512 && M <= 16 && K % 2048 == 0 ? 2 : 1;
   return 0;
 }
 
