@@ -398,7 +398,7 @@ def test_token_array_takes_tensors_of_one_element():
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch", [8, 9, 17, 32])
 def test_batch_step_on_both_sides_of_nine_rows(gpu_device, batch):
-    """From nine rows on a step's o, gate/up and down projections are panel GEMMs
+    """From nine rows on a step's o and down (from 17, gate/up) projections are panel GEMMs
     with the norm behind them: the first, middle and last sequence against the
     oracle, as the smaller batches are checked."""
     from tests.test_gpu_batch import _oracle_runs

@@ -103,3 +103,15 @@ def test_panel_gemm_slices_of_a_refused_shape_are_zero(M, K, N):
     from tilefoundry_amd._lib import lib
 
     assert lib().tfd_panel_gemm_slices(M, K, N) == 0
+
+
+@pytest.mark.parametrize("rows,inter,panels", [
+    (1, 6144, False), (16, 6144, False), (17, 6144, True), (32, 6144, True), (33, 6144, True),
+    (33, 9728, True), (16, 8192, False), (17, 8192, True), (32, 9728, False), (32, 12288, True),
+    (32, 5632, False), (4096, 768, True)])
+def test_gate_up_takes_panels_where_their_blocks_fill_the_chip(rows, inter, panels):
+    """256 compute units, blocks of 64 columns: 9,728 leaves the second round at a fifth,
+    5,632 the first at 176 of 256; up to 16 rows the skinny GEMM, past 32 always panels."""
+    from tilefoundry_amd.qwen3.prefill import gate_up_panels
+
+    assert gate_up_panels(rows, inter, 256) is panels

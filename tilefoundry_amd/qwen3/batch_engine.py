@@ -7,8 +7,8 @@ The batch-1 engine's structure (``engine.py``; the reference's
   shared page pool per layer (``[B * pages][HKV][16][D]`` bf16, a seeded
   permutation so every sequence's pages are scattered through the pool);
 * the projections are skinny GEMMs on the matrix cores
-  (``tfd_gemm_skinny_bf16``: M = batch rows, 16x16x32 bf16 MFMA; from nine rows on,
-  panel GEMMs whose sums the next norm adds), the norms run row by row, and
+  (``tfd_gemm_skinny_bf16``: M = batch rows, 16x16x32 bf16 MFMA; from nine rows on
+  o and down are panel GEMMs whose sums the next norm adds), the norms run row by row, and
   attention runs per (split, kv head, sequence);
 * the whole step -- every layer, the head, the per-sequence pick and the next
   embeddings -- is recorded once into a HIP graph and replayed; the last kernel
@@ -28,7 +28,8 @@ from .._lib import lib, ptr
 from ..sampling import Picker, Sampling
 from .config import Qwen3Config
 from .engine import bf16_scale, scatter_cache
-from .prefill import Prefill, attention_splits, in_vocab, int32_ids, token_array
+from .prefill import (Prefill, attention_splits, gate_up_panels, in_vocab, int32_ids,
+                      token_array)
 from .weights import head_rows, pack_layer, validate
 
 MAX_BATCH = 32
@@ -183,7 +184,11 @@ class BatchEngine:
         # next norm adds (as many launches, and no hand-off inside the GEMM).  A
         # step of eight layers of Qwen3-1.7B: 578 against 648 us at 32 rows, 534 / 553
         # at 16, 518 / 520 at 8; at one row 503 / 464, where the skinny GEMM wastes less.
+        # (Gate/up by ``gate_up_panels``: 16 rows 512 us, 12 rows 504 against 518.)
         self.panels = B > 8
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        self.panel_gu = (self._lib.tfd_panel_gemm_slices(B, self.H, 2 * self.I) == 1 and
+                         gate_up_panels(B, self.I, cus))
         self.part = z(max(self._lib.tfd_panel_gemm_slices(B, K, self.H) for K in
                           (self.QD, self.I)) * B * self.H, dtype=f32)
 
@@ -239,7 +244,7 @@ class BatchEngine:
             self._norm(x_out, gamma, s)
             return
         self._project(self.attn, w["w_o"], self.QD, x_in, self.h1, w["gamma_post"], s)
-        if L.tfd_panel_gemm_slices(B, H, 2 * I) == 1:
+        if self.panel_gu:
             L.tfd_panel_gemm_bf16(ptr(self.xn), ptr(w["w_gu"]), B, H, 2 * I, _lib.PANEL_SWIGLU,
                                   ptr(self.hmid), s)
         else:

@@ -49,6 +49,20 @@ def attention_splits(rows: int, kv_heads: int, cap: int) -> int:
     return max(1, min(tiles, -(-SPLIT_BLOCKS // (rows * kv_heads))))
 
 
+def gate_up_panels(rows: int, inter: int, cus: int) -> bool:
+    """Whether the gate/up projection of *rows* rows goes through the panel GEMM rather
+    than the skinny one (which takes up to 32).  The panel GEMM multiplies 32 rows
+    whatever their number, the skinny one 16 up to 16; and its blocks of 64 columns want
+    full rounds of the *cus* compute units.  Steps of three or four layers with the skinny
+    / the panel gate/up (hidden x inter, us): 16 rows 2,048 x 6,144 216 / 219, 4,096 x
+    12,288 (1.5 rounds of blocks) 297 / 320, 2,560 x 9,728 (1.2 rounds) 289 / 341; 24 rows
+    226 / 221, 318 / 325, 317 / 344; 32 rows 240 / 231, 343 / 335, 341 / 354."""
+    if rows <= 16 or rows > 32:
+        return rows > 32
+    blocks = -(-2 * inter // 64)
+    return 10 * blocks >= 7 * cus * -(-blocks // cus)
+
+
 def token_array(tokens) -> np.ndarray:
     """Token ids (any sequence of them) as an int64 array."""
     try:
@@ -166,6 +180,9 @@ class Prefill:
                 for n in ("w_qkv", "w_o", "w_gu", "w_down"):
                     lw[n] = self._mfma_order(w[n], s)
             self.layers.append(lw)
+        # the skinny GEMM's tile counters (kept at zero by the library) and partial tiles
+        self.work = torch.zeros(1 << 21, device=self.dev, dtype=torch.float32)
+        self.cus = torch.cuda.get_device_properties(self.dev).multi_processor_count
         torch.cuda.synchronize(self.dev)
         self.rows = 0
 
@@ -229,7 +246,12 @@ class Prefill:
         sl = self._gemm(self.attn, w["w_o"], M, self.QD, H, s)
         L.tfd_panel_add_norm(ptr(self.part), sl, ptr(self.hid), ptr(self.h1),
                              ptr(w["gamma_post"]), ptr(self.xn), M, H, self.eps, s)
-        if self._slices(M, H, 2 * I) == 1:
+        slices = self._slices(M, H, 2 * I)
+        if M <= 16 or not (slices > 1 or gate_up_panels(M, I, self.cus)):
+            L.tfd_gemm_skinny_bf16(ptr(self.xn), ptr(w["w_gu"]), M, H, 2 * I, _lib.EPI_SWIGLU,
+                                   None, 0, ptr(self.hmid), 0, ptr(self.work),
+                                   self.work.numel(), s)
+        elif slices == 1:
             L.tfd_panel_gemm_bf16(ptr(self.xn), ptr(w["w_gu"]), M, H, 2 * I, _lib.PANEL_SWIGLU,
                                   ptr(self.hmid), s)
         else:
