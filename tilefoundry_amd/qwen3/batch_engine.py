@@ -343,7 +343,7 @@ class BatchEngine:
         if len(prompts) != self.B or any(len(p) < 1 for p in prompts):
             raise ValueError(f"need {self.B} non-empty prompts")
         if getattr(self, "_prefiller", None) is None:
-            self._prefiller = Prefill(weakref.proxy(self), packed=True)
+            self._prefiller = Prefill(weakref.ref(self), packed=True)
         self._load_prompts(prompts)
         self._prefiller.run_many([(p[:-1], 0, b) for b, p in enumerate(prompts) if len(p) > 1])
         self.pos.copy_(torch.tensor([len(p) - 1 for p in prompts], dtype=torch.int32))

@@ -384,7 +384,7 @@ class Engine:
         if pl < 2:
             return
         if getattr(self, "_prefiller", None) is None:
-            self._prefiller = Prefill(weakref.proxy(self))    # no cycle: see its docstring
+            self._prefiller = Prefill(weakref.ref(self))
         self._prefiller.run(prompt_ids[:-1], 0)
         self.pos.fill_(pl - 1)
         self.ids.fill_(int(prompt_ids[-1]))

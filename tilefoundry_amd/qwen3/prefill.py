@@ -24,6 +24,7 @@ go through together.
 """
 from __future__ import annotations
 
+import weakref
 from array import array
 from operator import index
 
@@ -154,13 +155,13 @@ class Prefill:
     pool), ``cos``/``sin``, ``cap``).  With *packed* False the projections are
     re-laid once into the skinny GEMMs' operand blocks (one more copy of the
     layer weights in HBM); a batch engine's layers are already in that order.
-    An engine that keeps its own pass hands in a weak proxy of itself: with a cycle the
+    An engine that keeps its own pass hands in a weak reference to itself: with a cycle the
     device memory of both would stay until a garbage collection.  Workspaces grow to the
     largest pass seen, ``MAX_PASS`` rows at most."""
 
     def __init__(self, engine, packed: bool = False):
-        e = engine
-        self.e = e
+        self._engine = engine if isinstance(engine, weakref.ref) else lambda: engine
+        e = self.e
         self._lib = lib()
         self.dev = e.device
         self.L, self.H, self.I, self.D = e.L, e.H, e.I, e.D
@@ -185,6 +186,10 @@ class Prefill:
         self.cus = torch.cuda.get_device_properties(self.dev).multi_processor_count
         torch.cuda.synchronize(self.dev)
         self.rows = 0
+
+    @property
+    def e(self):
+        return self._engine()
 
     def _mfma_order(self, w, s):
         N, K = w.shape
